@@ -12,6 +12,7 @@
  *                           in host memory, passed in the kernel arguments).
  *   4. Paged prefill attn : packed new tokens of several sequences over their cached
  *                           prefixes and themselves, causal, reading K/V pages in place.
+ *   5. Layer elementwise  : residual add + RMS norm, and SiLU(gate) * up.
  *
  * Pool layout (one layer; identical to the reference pool
  * engine/kv_cache.py:426-428, `k, v: [num_layers, num_blocks + 1, num_kv_heads,
@@ -340,6 +341,26 @@ int mip_copy_blocks(void* k_cache, void* v_cache, const int64_t* pairs, int32_t 
 int mip_copy_blocks_host(void* k_cache, void* v_cache, const int64_t* pairs, int32_t n_pairs,
                          int32_t num_layers, int64_t num_cache_blocks, int64_t block_bytes,
                          void* stream);
+
+/*
+ * Residual add + RMS norm of `rows` contiguous rows of `dim` elements, one launch:
+ *     s   = rnd(x + delta)                       (s = x where delta is NULL)
+ *     out = rnd(weight * rnd(s * rsqrt(mean(s^2) + eps)))
+ * with sums and products in fp32 and rnd = round to nearest even into dtype, the values torch's
+ * op-by-op evaluation of engine/model.py's RMSNorm stores. `sum` receives s; it is NULL exactly
+ * when delta is, and may be x or delta itself. Rows whose byte length is no multiple of 16 or
+ * exceeds 32 KB, and addresses that are not 16-byte aligned, are MIP_EUNSUPPORTED.
+ */
+int mip_add_rms_norm(void* out, void* sum, const void* x, const void* delta, const void* weight,
+                     int32_t rows, int32_t dim, float eps, int32_t dtype, void* stream);
+
+/*
+ * The MLP's gating: out[r, j] = rnd(rnd(silu(gate_up[r, j])) * gate_up[r, inter + j]), j < inter,
+ * over contiguous rows (gate_up rows of 2 * inter elements), silu(g) = g / (1 + exp(-g)) in fp32.
+ * Rows whose byte length is no multiple of 16, unaligned addresses and 2^31 or more 16-byte
+ * chunks are MIP_EUNSUPPORTED.
+ */
+int mip_silu_mul(void* out, const void* gate_up, int32_t rows, int32_t inter, int32_t dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -47,6 +47,14 @@ template <> __device__ __forceinline__ float from_f32<MIP_F32>(float f) { return
 template <> __device__ __forceinline__ uint16_t from_f32<MIP_F16>(float f) { return f32_to_f16_rne(f); }
 template <> __device__ __forceinline__ uint16_t from_f32<MIP_BF16>(float f) { return f32_to_bf16_rne(f); }
 
+// An element as fp32 (exact), and the value a torch op on dtype tensors stores: fp32 rounded to
+// the dtype and back.
+template <int DT> __device__ __forceinline__ float widen(typename Elem<DT>::S s);
+template <> __device__ __forceinline__ float widen<MIP_F32>(float s) { return s; }
+template <> __device__ __forceinline__ float widen<MIP_F16>(uint16_t s) { return f16_bits_to_f32(s); }
+template <> __device__ __forceinline__ float widen<MIP_BF16>(uint16_t s) { return __uint_as_float(uint32_t{s} << 16); }
+template <int DT> __device__ __forceinline__ float rnd(float f) { return widen<DT>(from_f32<DT>(f)); }
+
 // 2-term dot product of packed 16-bit pairs accumulated in fp32 (v_dot2_f32_{bf16,f16}).
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));

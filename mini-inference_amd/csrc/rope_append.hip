@@ -44,14 +44,6 @@ struct RopeArgs {
   int n_tokens, hq, hkv, half_bytes, row_bytes, block_size, log2_bs;
 };
 
-template <int DT> __device__ __forceinline__ float widen(typename Elem<DT>::S s);
-template <> __device__ __forceinline__ float widen<MIP_F32>(float s) { return s; }
-template <> __device__ __forceinline__ float widen<MIP_F16>(uint16_t s) { return f16_bits_to_f32(s); }
-template <> __device__ __forceinline__ float widen<MIP_BF16>(uint16_t s) { return __uint_as_float(uint32_t{s} << 16); }
-
-// Round an fp32 value to the dtype and back (the value a torch op on dtype tensors stores).
-template <int DT> __device__ __forceinline__ float rnd(float f) { return widen<DT>(from_f32<DT>(f)); }
-
 // fp32 multiply and add that are never contracted into an fma (each rounds on its own, as
 // torch's separate elementwise kernels do).
 __device__ __forceinline__ float mul_rn(float a, float b) {

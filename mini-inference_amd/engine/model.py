@@ -4,8 +4,10 @@ The attention layer hands its post-RoPE q, k, v to an ``AttentionContext`` and g
 attention output back, exactly as engine/model.py:241-251 of the reference does
 (``out = ctx.attend(self.layer_idx, q, k, v)``). The cache contexts in
 :mod:`engine.kv_cache` implement that protocol with the HIP kernels; this module only
-supplies the surrounding projections, norms, RoPE and MLP in PyTorch so that a full
-decode step can be timed with random-init weights (no checkpoint is loaded).
+supplies the surrounding projections, norms, RoPE and MLP so that a full decode step can be
+timed with random-init weights (no checkpoint is loaded). Norms, residual adds and the MLP's
+gating run as fused kernels (:mod:`engine.layer_ops`) in inference on the GPU and as torch ops
+everywhere else.
 
 Shapes (reference engine/model.py:89-98): q ``[B, Hq, T, D]``, k and v
 ``[B, Hkv, T, D]``; ``attend`` returns ``[B, Hq, T, D]``.
@@ -20,6 +22,8 @@ from typing import Protocol
 import torch
 import torch.nn.functional as F
 from torch import nn
+
+from . import layer_ops
 
 
 @dataclass(frozen=True)
@@ -71,6 +75,18 @@ class AttentionContext(Protocol):
     def attend(self, layer_idx: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor: ...
 
 
+def _plain(module: nn.Module, cls: type) -> bool:
+    """Whether calling ``module`` does what ``cls.forward`` says and nothing else: its exact class, no hooks.
+
+    A fused step that passes a submodule's call by is only taken where nobody watches that call.
+    """
+    g = nn.modules.module
+    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
+            and not module._forward_pre_hooks and not module._backward_hooks and not module._backward_pre_hooks
+            and not g._global_forward_hooks and not g._global_forward_pre_hooks and not g._global_backward_hooks
+            and not g._global_backward_pre_hooks)
+
+
 class RMSNorm(nn.Module):
     """x / rms(x) * weight with the statistic taken in fp32, result cast back first."""
 
@@ -80,6 +96,8 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if layer_ops.norm_usable(self.weight, x):
+            return layer_ops.rms_norm(x, self.weight, self.eps)
         xf = x.float()
         inv = torch.rsqrt(xf.square().mean(dim=-1, keepdim=True) + self.eps)
         return self.weight * (xf * inv).to(x.dtype)
@@ -133,7 +151,10 @@ class MLP(nn.Module):
         self.down_proj = nn.Linear(cfg.intermediate_size, cfg.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        gate, up = self.gate_up_proj(x).chunk(2, dim=-1)
+        gate_up = self.gate_up_proj(x)
+        if layer_ops.silu_mul_usable(gate_up):
+            return self.down_proj(layer_ops.silu_mul(gate_up))
+        gate, up = gate_up.chunk(2, dim=-1)
         return self.down_proj(F.silu(gate) * up)
 
 
@@ -146,7 +167,11 @@ class DecoderLayer(nn.Module):
         self.mlp = MLP(cfg)
 
     def forward(self, x, cos, sin, ctx):
-        x = x + self.attn(self.input_norm(x), cos, sin, ctx)
+        delta, norm = self.attn(self.input_norm(x), cos, sin, ctx), self.post_attn_norm
+        if _plain(norm, RMSNorm) and layer_ops.norm_usable(norm.weight, x, delta):
+            x, normed = layer_ops.add_rms_norm(x, delta, norm.weight, norm.eps)
+            return x + self.mlp(normed)
+        x = x + delta
         return x + self.mlp(self.post_attn_norm(x))
 
 

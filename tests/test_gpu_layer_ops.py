@@ -1,0 +1,145 @@
+"""Fused layer kernels against float64 restatements, and the routes that must stay on torch ops."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+# Unit roundoff of each dtype: an output that passes n roundings is within n * U of the 64-bit value.
+U = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+TINY = 2.0 ** -24  # fp16 subnormal grid (absolute), far below everything else
+
+
+def norm64(s, w, eps):
+    s = s.double()
+    return w.double() * s * torch.rsqrt(s.square().mean(-1, keepdim=True) + eps)
+
+
+# Row lengths at every edge of the kernel's (wavefronts per row, chunks per lane) choices, in 16-byte
+# chunks: 1, 63, 112 (0.5B), 128 | 129, 256 | 257, 448 (7B), 512 | 513, 1024 | 1025, 2048.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("chunks", [1, 63, 112, 128, 129, 256, 257, 448, 512, 513, 1024, 1025, 2048])
+def test_add_rms_norm(gpu, dtype, chunks):
+    from engine import layer_ops
+
+    dim = chunks * 128 // torch.finfo(dtype).bits
+    for rows in (1, 3, 4, 517):
+        announce(f"add_rms_norm {dtype} rows {rows} dim {dim}")
+        gen = torch.Generator(device=gpu).manual_seed(rows + dim)
+        x = torch.randn(2, rows, dim, generator=gen, device=gpu).to(dtype)[1]
+        d = torch.randn(rows, dim, generator=gen, device=gpu).to(dtype)
+        w = (torch.rand(dim, generator=gen, device=gpu) + 0.5).to(dtype)
+        assert layer_ops.norm_usable(w, x, d)
+        s, h = layer_ops.add_rms_norm(x, d, w, 1e-6)
+        assert torch.equal(s, x + d)
+        only = layer_ops.rms_norm(x, w, 1e-6)
+        # Two roundings (three for 32 bits, whose sum of dim squares is also within dim * U, in
+        # practice far less: 64 lanes add dim / 64 terms each), and rsqrt's last bit.
+        slack = 2.05 * U[dtype] + (dim / 64 + 16) * U[torch.float32]
+        for got, src in ((h, s), (only, x)):
+            want = norm64(src, w, 1e-6)
+            assert ((got.double() - want).abs() <= slack * want.abs() + TINY).all()
+
+
+def test_rms_norm_special_values(gpu):
+    from engine import layer_ops
+
+    announce("rms_norm with zero, infinite and NaN rows")
+    x = torch.randn(4, 896, device=gpu).to(torch.bfloat16)
+    x[0] = 0
+    x[1, 5] = float("inf")
+    x[2, 7] = float("nan")
+    w = torch.ones(896, device=gpu, dtype=torch.bfloat16)
+    got = layer_ops.rms_norm(x, w, 1e-6)
+    xf = x.float()
+    want = w * (xf * torch.rsqrt(xf.square().mean(-1, keepdim=True) + 1e-6)).to(x.dtype)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1].nan_to_num(7.0), want[1].nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,inter", [(1, 8), (3, 4864), (257, 264), (70, 18944)])
+def test_silu_mul(gpu, dtype, rows, inter):
+    from engine import layer_ops
+
+    announce(f"silu_mul {dtype} rows {rows} inter {inter}")
+    x = (4 * torch.randn(rows, 2 * inter, device=gpu)).to(dtype)
+    x[0, :4] = torch.tensor([60.0, -60.0, 0.0, -20.0], device=gpu).to(dtype)
+    assert layer_ops.silu_mul_usable(x)
+    got = layer_ops.silu_mul(x)
+    g, u = x.double().chunk(2, dim=-1)
+    want = g * torch.sigmoid(g) * u
+    # Two roundings, and a few fp32 roundings of exp, the sum and the quotient (exp's argument
+    # rounding is exact, its result within 2 ulps).
+    slack = 2.05 * U[dtype] + 8 * U[torch.float32]
+    assert ((got.double() - want).abs() <= slack * want.abs() + TINY * (1 + u.abs())).all()
+
+
+def test_routes_that_stay_on_torch(gpu):
+    """Calls that something observes, and layouts the kernels do not take, keep the torch ops and their results."""
+    from engine import layer_ops
+    from engine.model import MLP, DecoderLayer, Qwen2Config, RMSNorm
+
+    announce("layer ops routing")
+    norm = RMSNorm(64, 1e-6).to(gpu)
+    x = torch.randn(6, 64, device=gpu)
+    with torch.no_grad():
+        want = norm(x)
+        assert layer_ops.norm_usable(norm.weight, x)
+    # autograd: same value, gradients flow to x and the weight
+    xg = x.clone().requires_grad_()
+    assert not layer_ops.norm_usable(norm.weight, xg)
+    y = norm(xg)
+    y.square().sum().backward()
+    assert xg.grad is not None and norm.weight.grad is not None
+    torch.testing.assert_close(y.detach(), want, rtol=1e-6, atol=1e-6)
+    with torch.no_grad():
+        # torch.func transforms and forward-mode AD
+        torch.testing.assert_close(torch.func.vmap(norm)(x), want, rtol=1e-6, atol=1e-6)
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+            assert not layer_ops.norm_usable(norm.weight, dual)
+        # unaligned, strided, ragged and mixed-dtype operands
+        odd = torch.randn(6 * 64 + 1, device=gpu)[1:].view(6, 64)
+        assert not layer_ops.norm_usable(norm.weight, odd) and norm(odd).shape == odd.shape
+        strided = torch.randn(64, 6, device=gpu).t()
+        assert not layer_ops.norm_usable(norm.weight, strided)
+        torch.testing.assert_close(norm(strided), norm(strided.contiguous()), rtol=1e-6, atol=1e-6)
+        assert not layer_ops.norm_usable(norm.weight, x.to(torch.bfloat16))
+        assert not layer_ops.norm_usable(norm.weight, x[:, :6])
+        assert not layer_ops.norm_usable(norm.weight, x, x[:1])  # a delta that would broadcast
+        assert norm(x[:0]).shape == (0, 64)
+        assert not layer_ops.silu_mul_usable(torch.randn(3, 12, device=gpu))
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert not layer_ops.norm_usable(norm.weight, x)
+
+    # A hook on the layer's second norm still sees its call.
+    cfg = Qwen2Config(vocab_size=64, hidden_size=64, intermediate_size=128, num_layers=1, num_heads=2, num_kv_heads=1,
+                      head_dim=32)
+    layer = DecoderLayer(cfg, 0).to(gpu).requires_grad_(False)
+
+    class Same:
+        def attend(self, layer_idx, q, k, v):
+            return q
+
+    cs = torch.ones(1, 1, 5, 32, device=gpu)
+    h = torch.randn(1, 5, 64, device=gpu)
+    with torch.inference_mode():
+        plain = layer(h, cs, cs * 0, Same())
+        seen = []
+        layer.post_attn_norm.register_forward_hook(lambda m, a, o: seen.append((a[0], o)))
+        hooked = layer(h, cs, cs * 0, Same())
+    assert len(seen) == 1 and seen[0][0].shape == h.shape
+    torch.testing.assert_close(hooked, plain, rtol=1e-5, atol=1e-6)
+    mlp = MLP(cfg).to(gpu)
+    a = torch.randn(3, 64, device=gpu, requires_grad=True)
+    mlp(a).sum().backward()
+    with torch.no_grad():
+        g, u = mlp.gate_up_proj(a).chunk(2, dim=-1)
+        torch.testing.assert_close(mlp(a), mlp.down_proj(F.silu(g) * u), rtol=1e-5, atol=1e-6)
+    assert a.grad is not None

@@ -13,6 +13,7 @@
  *   4. Paged prefill attn : packed new tokens of several sequences over their cached
  *                           prefixes and themselves, causal, reading K/V pages in place.
  *   5. Layer elementwise  : residual add + RMS norm, and SiLU(gate) * up.
+ *   6. Small linear       : linear layers of a decode step with norm, bias, residual or gating fused.
  *
  * Pool layout (one layer; identical to the reference pool
  * engine/kv_cache.py:426-428, `k, v: [num_layers, num_blocks + 1, num_kv_heads,
@@ -361,6 +362,24 @@ int mip_add_rms_norm(void* out, void* sum, const void* x, const void* delta, con
  * chunks are MIP_EUNSUPPORTED.
  */
 int mip_silu_mul(void* out, const void* gate_up, int32_t rows, int32_t inter, int32_t dtype, void* stream);
+
+/*
+ * Linear layers of a few rows (m <= 256; 16-bit dtypes), fused with the elementwise work beside
+ * them. Rows and weights are contiguous, weight[n][k] as torch's nn.Linear keeps it; products
+ * accumulate in fp32, rnd = round to nearest even into dtype.
+ *
+ * mip_norm_linear:     h   = rnd(norm * rnd(x * rsqrt(mean(x^2) + eps)))       [m][k]
+ *                      out = rnd(h weight^T + bias)                            [m][n]  (bias may be NULL)
+ *   with gate_up != 0: y   = rnd(h weight^T), out = rnd(rnd(silu(y[:, :n/2])) * y[:, n/2:])   [m][n/2]  (bias NULL)
+ * mip_linear_residual: out = rnd(residual + rnd(a weight^T))                   [m][n]; out may be residual
+ *
+ * n must be a multiple of 16 and k of 32, every address 16-byte aligned; other calls are
+ * MIP_EUNSUPPORTED.
+ */
+int mip_norm_linear(void* out, const void* x, const void* norm, float eps, const void* weight, const void* bias,
+                    int32_t m, int32_t n, int32_t k, int32_t gate_up, int32_t dtype, void* stream);
+int mip_linear_residual(void* out, const void* a, const void* weight, const void* residual, int32_t m,
+                        int32_t n, int32_t k, int32_t dtype, void* stream);
 
 #ifdef __cplusplus
 }

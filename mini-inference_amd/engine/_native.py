@@ -34,6 +34,8 @@ EXPORTED = (
     "mip_copy_blocks_host",
     "mip_add_rms_norm",
     "mip_silu_mul",
+    "mip_norm_linear",
+    "mip_linear_residual",
 )
 
 # Measurement helpers in the same library (include/mipaged_probe.h), outside the drop-in ABI.
@@ -87,6 +89,8 @@ _SIGNATURES = {
     "mip_copy_blocks_host": (_c.c_int, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp]),
     "mip_add_rms_norm": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _f32, _i32, _vp]),
     "mip_silu_mul": (_c.c_int, [_vp, _vp, _i32, _i32, _i32, _vp]),
+    "mip_norm_linear": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
+    "mip_linear_residual": (_c.c_int, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp]),
     "mip_hbm_read_probe": (_c.c_int, [_vp, _i64, _vp, _i64, _i32, _vp, _i32, _i32, _vp]),
 }
 

@@ -1,4 +1,4 @@
-"""Fused elementwise kernels of a decoder layer, used by :mod:`engine.model` where they apply.
+"""Fused kernels of a decoder layer, used by :mod:`engine.model` where they apply.
 
 ``usable`` is the rule: plain contiguous tensors of one supported dtype on the current ROCm
 device, with nothing recording, transforming or tracing the call. Everything else (CPU tensors,
@@ -93,4 +93,69 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
                                      _DTYPE_CODES[gate_up.dtype], _stream_ptr(gate_up.device))
     if st:
         _native.check(st, "mip_silu_mul")
+    return out
+
+
+# Where the fused linear kernels beat the library's product and the separate kernels around it: a
+# workgroup reads its rows of the input again for every 16 to 64 weight rows, so they win while
+# the rows are few or the weight small. Lines between measured shapes (bf16, weights cold, graph
+# replay, us, fused against library), n x k by rows:
+#   norm + linear     1152 x 896: 4.5/8.6 at 8 rows, 5.7/11.2 at 64, 10.1/11.2 at 256;
+#                     2560 x 2048: 8.8/16.2 at 16, 13.2/16.6 at 65, 26.4/19.7 at 128;
+#                     2048 x 1536: 12.7/13.8 at 128, 15.5/14.6 at 256; 4608 x 3584: 20.0/16.4 at 8
+#   norm + gate + up  9728 x 896: 9.3/14.6 at 8, 16.3/18.3 at 64, 27.0/18.4 at 65;
+#                     17920 x 1536: 28.7/47.4 at 16, 35.7/26.1 at 32; 22016 x 2048: 37.4/52.4 at 16;
+#                     37888 x 3584: 104/65 at 8
+#   linear + residual 896 x 896: 3.8/8.5 at 8, 6.2/9.7 at 256; 896 x 4864: 10.5/20.3 at 8,
+#                     12.0/19.1 at 64, 17.8/15.5 at 96; 2048 x 2048: 11.7/13.8 at 64;
+#                     3584 x 3584: 10.9/15.1 at 16, 18.7/14.9 at 32; 3584 x 18944: 39.0/48.7 at 16
+_HALF = (torch.float16, torch.bfloat16)
+
+
+def _linear_fits(rows: int, weight: torch.Tensor) -> bool:
+    n, k = weight.shape
+    return rows <= 256 and weight.dtype in _HALF and n % 16 == 0 and k % 32 == 0
+
+
+def norm_linear_pays(rows: int, weight: torch.Tensor) -> bool:
+    limit = 8 << 20 if rows <= 16 else 4 << 20 if rows <= 96 else 3 << 19
+    return _linear_fits(rows, weight) and weight.numel() <= limit
+
+
+def norm_gate_up_pays(rows: int, weight: torch.Tensor) -> bool:
+    limit = 48 << 20 if rows <= 16 else 12 << 20 if rows <= 64 else 0
+    return _linear_fits(rows, weight) and weight.numel() <= limit
+
+
+def linear_residual_pays(rows: int, weight: torch.Tensor) -> bool:
+    if not _linear_fits(rows, weight):
+        return False
+    return rows <= 16 or weight.numel() <= (5 << 20 if rows <= 64 else 1 << 20)
+
+
+def norm_linear(x: torch.Tensor, norm: torch.Tensor, eps: float, weight: torch.Tensor, bias: torch.Tensor | None = None,
+                gate_up: bool = False) -> torch.Tensor:
+    """The RMS norm of x's rows through a linear layer, in one launch.
+
+    With ``gate_up`` the weight holds gate rows, then as many up rows, and the result is
+    ``silu(gate) * up``.
+    """
+    n, k = weight.shape
+    out = torch.empty((*x.shape[:-1], n // 2 if gate_up else n), dtype=x.dtype, device=x.device)
+    st = _native.load().mip_norm_linear(out.data_ptr(), x.data_ptr(), norm.data_ptr(), eps, weight.data_ptr(),
+                                        None if bias is None else bias.data_ptr(), x.numel() // k, n, k, int(gate_up),
+                                        _DTYPE_CODES[x.dtype], _stream_ptr(x.device))
+    if st:
+        _native.check(st, "mip_norm_linear")
+    return out
+
+
+def linear_residual(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
+    """``residual + a @ weight.T`` in one launch."""
+    n, k = weight.shape
+    out = torch.empty_like(residual)
+    st = _native.load().mip_linear_residual(out.data_ptr(), a.data_ptr(), weight.data_ptr(), residual.data_ptr(),
+                                            a.numel() // k, n, k, _DTYPE_CODES[a.dtype], _stream_ptr(a.device))
+    if st:
+        _native.check(st, "mip_linear_residual")
     return out

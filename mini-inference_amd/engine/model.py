@@ -129,9 +129,13 @@ class Attention(nn.Module):
         self.o_proj = nn.Linear(cfg.q_size, cfg.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, ctx: AttentionContext) -> torch.Tensor:
+        return self.o_proj(self.attend(self.qkv_proj(x), cos, sin, ctx))
+
+    def attend(self, qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, ctx: AttentionContext) -> torch.Tensor:
+        """The part between the projections: ``[B, T, q + 2 kv]`` in, ``[B, T, q]`` out."""
         c = self.cfg
-        bsz, t, _ = x.shape
-        q, k, v = self.qkv_proj(x).split([c.q_size, c.kv_size, c.kv_size], dim=-1)
+        bsz, t, _ = qkv.shape
+        q, k, v = qkv.split([c.q_size, c.kv_size, c.kv_size], dim=-1)
         q = q.view(bsz, t, c.num_heads, c.head_dim).transpose(1, 2)
         k = k.view(bsz, t, c.num_kv_heads, c.head_dim).transpose(1, 2)
         v = v.view(bsz, t, c.num_kv_heads, c.head_dim).transpose(1, 2)
@@ -141,7 +145,7 @@ class Attention(nn.Module):
         else:
             q, k = apply_rope(q, k, cos, sin)
             out = ctx.attend(self.layer_idx, q, k, v)  # the call site the cache contexts serve
-        return self.o_proj(out.transpose(1, 2).reshape(bsz, t, c.q_size))
+        return out.transpose(1, 2).reshape(bsz, t, c.q_size)
 
 
 class MLP(nn.Module):
@@ -151,11 +155,14 @@ class MLP(nn.Module):
         self.down_proj = nn.Linear(cfg.intermediate_size, cfg.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        gate_up = self.gate_up_proj(x)
+        return self.down_proj(self.gated(self.gate_up_proj(x)))
+
+    @staticmethod
+    def gated(gate_up: torch.Tensor) -> torch.Tensor:
         if layer_ops.silu_mul_usable(gate_up):
-            return self.down_proj(layer_ops.silu_mul(gate_up))
+            return layer_ops.silu_mul(gate_up)
         gate, up = gate_up.chunk(2, dim=-1)
-        return self.down_proj(F.silu(gate) * up)
+        return F.silu(gate) * up
 
 
 class DecoderLayer(nn.Module):
@@ -167,12 +174,61 @@ class DecoderLayer(nn.Module):
         self.mlp = MLP(cfg)
 
     def forward(self, x, cos, sin, ctx):
-        delta, norm = self.attn(self.input_norm(x), cos, sin, ctx), self.post_attn_norm
-        if _plain(norm, RMSNorm) and layer_ops.norm_usable(norm.weight, x, delta):
-            x, normed = layer_ops.add_rms_norm(x, delta, norm.weight, norm.eps)
-            return x + self.mlp(normed)
-        x = x + delta
+        if self._fusable(x):
+            x, delta = self._fused(x, None, cos, sin, ctx)
+            return x if delta is None else x + delta
+        x = x + self.attn(self.input_norm(x), cos, sin, ctx)
         return x + self.mlp(self.post_attn_norm(x))
+
+    def _fusable(self, x: torch.Tensor) -> bool:
+        """Whether the layer may run as its fused steps: unwatched submodules, operands the kernels take."""
+        a, m, n1, n2 = self.attn, self.mlp, self.input_norm, self.post_attn_norm
+        if not (_plain(n1, RMSNorm) and _plain(n2, RMSNorm) and _plain(a, Attention) and _plain(m, MLP)):
+            return False
+        linears = (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj)
+        if not all(_plain(p, nn.Linear) for p in linears) or any(p.bias is not None for p in linears[1:]):
+            return False
+        w = [p.weight for p in linears] + ([a.qkv_proj.bias] if a.qkv_proj.bias is not None else [])
+        h = x.shape[-1]
+        return (x.dim() == 3 and w[0].shape[1] == h and w[1].shape[0] == h and w[2].shape[1] == h
+                and w[3].shape == (h, w[2].shape[0] // 2) and n2.weight.shape == n1.weight.shape
+                and layer_ops.norm_usable(n1.weight, x) and layer_ops.usable(x, n2.weight, *w))
+
+    def _fused(self, x, delta, cos, sin, ctx):
+        """``forward`` of ``x + delta`` (None: of x), as ``(y, delta)`` whose sum it is (None: y is).
+
+        Norms, bias, residual adds and gating run inside the linear layers where rows are few, and
+        as one kernel each between library products where they are many; there the last residual
+        add is left to the caller, which may have a norm to fuse it with.
+        """
+        a, m, n1, n2 = self.attn, self.mlp, self.input_norm, self.post_attn_norm
+        rows = x.shape[0] * x.shape[1]
+        w = a.qkv_proj.weight
+        if delta is not None:
+            x, normed = layer_ops.add_rms_norm(x, delta, n1.weight, n1.eps)
+            qkv = F.linear(normed, w, a.qkv_proj.bias)
+        elif layer_ops.norm_linear_pays(rows, w):
+            qkv = layer_ops.norm_linear(x, n1.weight, n1.eps, w, a.qkv_proj.bias)
+        else:
+            qkv = F.linear(layer_ops.rms_norm(x, n1.weight, n1.eps), w, a.qkv_proj.bias)
+        out, w = a.attend(qkv, cos, sin, ctx), a.o_proj.weight
+        if out.shape[:2] != x.shape[:2] or not layer_ops.usable(x, out):  # a context with outputs of its own kind
+            x = x + F.linear(out, w)
+            return x + m(n2(x)), None
+        w2 = m.gate_up_proj.weight
+        if layer_ops.linear_residual_pays(rows, w):
+            x = layer_ops.linear_residual(out, w, x)
+            normed = None if layer_ops.norm_gate_up_pays(rows, w2) else layer_ops.rms_norm(x, n2.weight, n2.eps)
+        else:
+            x, normed = layer_ops.add_rms_norm(x, F.linear(out, w), n2.weight, n2.eps)
+        if normed is None:
+            act = layer_ops.norm_linear(x, n2.weight, n2.eps, w2, gate_up=True)
+        else:
+            act = m.gated(F.linear(normed, w2))
+        w = m.down_proj.weight
+        if layer_ops.linear_residual_pays(rows, w) and layer_ops.usable(x, act):
+            return layer_ops.linear_residual(act, w, x), None
+        return x, F.linear(act, w)
 
 
 class Qwen2ForCausalLM(nn.Module):
@@ -189,9 +245,17 @@ class Qwen2ForCausalLM(nn.Module):
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, ctx: AttentionContext) -> torch.Tensor:
         x = self.embed_tokens(input_ids)
         cos, sin = rope_cos_sin(positions, self.cfg.head_dim, self.cfg.rope_theta, x.dtype)
+        delta = None  # the last fused layer's residual add, left for the norm that follows it
         for layer in self.layers:
-            x = layer(x, cos, sin, ctx)
-        return self.norm(x)
+            if _plain(layer, DecoderLayer) and layer._fusable(x):
+                x, delta = layer._fused(x, delta, cos, sin, ctx)
+            else:
+                x, delta = layer(x if delta is None else x + delta, cos, sin, ctx), None
+        if delta is None:
+            return self.norm(x)
+        if _plain(self.norm, RMSNorm) and layer_ops.norm_usable(self.norm.weight, x, delta):
+            return layer_ops.add_rms_norm(x, delta, self.norm.weight, self.norm.eps)[1]
+        return self.norm(x + delta)
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         w = self.embed_tokens.weight if self.lm_head is None else self.lm_head.weight

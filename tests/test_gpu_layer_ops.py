@@ -143,3 +143,95 @@ def test_routes_that_stay_on_torch(gpu):
         g, u = mlp.gate_up_proj(a).chunk(2, dim=-1)
         torch.testing.assert_close(mlp(a), mlp.down_proj(F.silu(g) * u), rtol=1e-5, atol=1e-6)
     assert a.grad is not None
+
+
+# Rows at the edges of the row tiles (16, 32, 64, 128, 256) and of each kernel's tile choice; widths that
+# leave a single 16-column tile, an odd number of tiles, fewer k-steps than wavefronts, k-steps that do
+# not divide among them, and the 0.5B model's own shapes.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(16, 32), (48, 96), (80, 1056), (1152, 896), (896, 4864), (2080, 160)])
+def test_small_linears(gpu, dtype, n, k):
+    from engine import layer_ops
+
+    for m in (1, 15, 16, 17, 32, 33, 64, 65, 128, 129, 200, 256):
+        announce(f"small linears {dtype} m {m} n {n} k {k}")
+        gen = torch.Generator(device=gpu).manual_seed(m * n + k)
+        x = torch.randn(1, m, k, generator=gen, device=gpu).to(dtype)
+        w = (torch.randn(n, k, generator=gen, device=gpu) / k ** 0.5).to(dtype)
+        norm = (torch.rand(k, generator=gen, device=gpu) + 0.5).to(dtype)
+        bias = torch.randn(n, generator=gen, device=gpu).to(dtype)
+        res = torch.randn(1, m, n, generator=gen, device=gpu).to(dtype)
+        xd, wd, u = x.double(), w.double(), U[dtype]
+        # Roundings of the product and of the result, fp32 sums of k products (their worst case), and
+        # with the norm two roundings of each of its elements: an error of independent terms, whose
+        # deviation is below U times the root of their squares' sum; 8 deviations.
+        got = layer_ops.linear_residual(x, w, res)
+        y = xd @ wd.t()
+        mag = xd.abs() @ wd.abs().t()
+        want = y + res.double()
+        assert ((got.double() - want).abs() <= 1.01 * u * (want.abs() + y.abs()) + (k / 64 + 8) * 2 ** -24 * mag + TINY).all()
+        h = norm64(x, norm, 1e-6)
+        y = h @ wd.t()
+        spread = (h.square() @ wd.square().t()).sqrt()
+        got = layer_ops.norm_linear(x, norm, 1e-6, w, bias)
+        want = y + bias.double()
+        assert ((got.double() - want).abs() <= 1.01 * u * want.abs() + 8 * u * spread + TINY).all()
+        bare = layer_ops.norm_linear(x, norm, 1e-6, w)
+        assert ((bare.double() - y).abs() <= 1.01 * u * y.abs() + 8 * u * spread + TINY).all()
+        got = layer_ops.norm_linear(x, norm, 1e-6, w, gate_up=True)
+        g, up = y.chunk(2, dim=-1)
+        sg, su = spread.chunk(2, dim=-1)
+        want = g * torch.sigmoid(g) * up  # |silu'| <= 1.1
+        slack = 8 * u * (1.1 * sg * (up.abs() + 8 * u * su) + g.abs() * su)
+        slack += u * (1.2 * g.abs() * up.abs() + want.abs())  # gate and up are rounded before their product
+        assert ((got.double() - want).abs() <= 2.02 * u * want.abs() + slack + TINY).all()
+
+
+def test_small_linears_refuse_what_they_do_not_take(gpu):
+    from engine import _native
+
+    announce("small linears: host checks")
+    lib, t = _native.load(), torch.zeros(64, 64, device=gpu, dtype=torch.bfloat16)
+    p = t.data_ptr()
+    assert lib.mip_linear_residual(p, p, p, p, 257, 16, 32, 2, None) == _native.MIP_EUNSUPPORTED
+    assert lib.mip_linear_residual(p, p, p, p, 1, 24, 32, 2, None) == _native.MIP_EUNSUPPORTED
+    assert lib.mip_linear_residual(p, p, p, p, 1, 16, 48, 2, None) == _native.MIP_EUNSUPPORTED
+    assert lib.mip_linear_residual(p, p, p, p, 1, 16, 32, 0, None) == _native.MIP_EUNSUPPORTED
+    assert lib.mip_linear_residual(p + 2, p, p, p, 1, 16, 32, 2, None) == _native.MIP_EUNSUPPORTED
+    assert lib.mip_linear_residual(p, p, p, None, 1, 16, 32, 2, None) == _native.MIP_EINVAL
+    assert lib.mip_norm_linear(p, p, None, 1e-6, p, None, 1, 16, 32, 0, 2, None) == _native.MIP_EINVAL
+    assert lib.mip_norm_linear(p, p, p, 1e-6, p, p, 1, 16, 32, 1, 2, None) == _native.MIP_EINVAL
+    assert lib.mip_linear_residual(p, p, p, p, 0, 16, 32, 2, None) == _native.MIP_OK
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_fused_layer_matches_its_modules(gpu, dtype):
+    """A layer through its fused steps against the same layer with a hook (which keeps the modules' own calls)."""
+    from engine.model import DecoderLayer, Qwen2Config
+
+    class Same:
+        def attend(self, layer_idx, q, k, v):
+            return q
+
+    # (hidden, intermediate): the kernels' shapes, and a width with k % 32 != 0 that stays on the library.
+    for hidden, inter in ((64, 128), (896, 4864), (72, 144)):
+        cfg = Qwen2Config(vocab_size=64, hidden_size=hidden, intermediate_size=inter, num_layers=1, num_heads=hidden // 8,
+                          num_kv_heads=1, head_dim=8)
+        layer = DecoderLayer(cfg, 0).to(gpu).to(dtype).requires_grad_(False)
+        layer.attn.qkv_proj.weight.mul_(2.0)
+        for b, t in ((1, 1), (8, 1), (1, 17), (64, 1), (65, 1), (2, 100), (1, 300)):
+            announce(f"fused layer {dtype} hidden {hidden} {b} x {t}")
+            x = torch.randn(b, t, hidden, device=gpu).to(dtype)
+            keep = x.clone()
+            cs = torch.ones(b, 1, t, 8, device=gpu, dtype=dtype)
+            with torch.inference_mode():
+                assert layer._fusable(x)
+                got = layer(x, cs, cs * 0, Same())
+                handle = layer.mlp.register_forward_hook(lambda m, a, o: None)
+                assert not layer._fusable(x)
+                want = layer(x, cs, cs * 0, Same())
+                handle.remove()
+            assert torch.equal(x, keep)  # the input is not written
+            # Both round each intermediate once or twice: a few roundings of relative size U each.
+            err = (got.double() - want.double()).norm() / want.double().norm()
+            assert err <= 8 * U[dtype], (hidden, b, t, float(err))

@@ -671,11 +671,13 @@ __global__ __launch_bounds__(256) void paged_decode_merge(DecodeArgs a) {
 
 inline int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
-enum class Algo { kValu, kMfma, kStream };
+enum class Algo { kValu, kMfma, kStream, kF32 };
 
 bool mfma_eligible(int dtype, int d, int g) {
   return (dtype == MIP_BF16 || dtype == MIP_F16) && (d == 64 || d == 128) && g >= 1 && g <= 16;
 }
+
+bool f32_eligible(int dtype, int d, int g) { return dtype == MIP_F32 && (d == 64 || d == 128) && g >= 1 && g <= 16; }
 
 // Forced algorithm (mip_set_decode_algo; MIP_ALGO_AUTO = the default choice below). Its
 // first value comes from MIP_DECODE_ALGO=valu|mfma|stream, read once.
@@ -691,19 +693,22 @@ std::atomic<int>& forced_algo() {
 
 // Default: the stream-K MFMA kernel for 16-bit data at head_dim 64/128 (balanced persistent
 // work split, the fastest under rocprof at the Qwen shapes) while its per-sequence scan fits
-// in LDS (batch <= 4096); otherwise the per-partition MFMA kernel; the VALU kernel for fp32
-// and the other head sizes. A forced algorithm applies where its kernel exists.
+// in LDS (batch <= 4096); otherwise the per-partition MFMA kernel; for fp32 at head_dim 64/128 the
+// fp32 MFMA kernel; the VALU kernel for the other head sizes and for groups of more than 16
+// heads. A forced algorithm applies where its kernel exists.
 Algo choose_algo(int dtype, int d, int g, int batch) {
   const int f = forced_algo().load(std::memory_order_relaxed);
   const bool mfma_ok = mfma_eligible(dtype, d, g);
   const bool stream_ok = mfma_ok && stream_config(dtype, d, g, batch).ok;
   if (f == MIP_ALGO_VALU) return Algo::kValu;
+  if (f32_eligible(dtype, d, g)) return Algo::kF32;
   if (f == MIP_ALGO_MFMA && mfma_ok) return Algo::kMfma;
   if (f == MIP_ALGO_STREAM && stream_ok) return Algo::kStream;
   return stream_ok ? Algo::kStream : mfma_ok ? Algo::kMfma : Algo::kValu;
 }
 
 int pass_tokens(Algo algo, int dtype, int d) {
+  if (algo == Algo::kF32) return 16;
   if (algo != Algo::kValu) return d <= 64 ? 32 : 16;
   const int es = dtype == MIP_F32 ? 4 : 2;
   const int ch = d < 32 / es ? d : 32 / es;
@@ -772,7 +777,6 @@ int valu_heads(int g) {
   return (g + s - 1) / s;
 }
 
-using KernelFn = void (*)(DecodeArgs);
 struct KernelPair {
   KernelFn part = nullptr;
   KernelFn merge = nullptr;
@@ -848,7 +852,31 @@ KernelPair pick_mfma_d(int d, int g) {
   }
 }
 
+template <int D>
+KernelFn pick_f32_merge(int g) {
+  switch (g) {
+    case 1: return paged_decode_merge<MIP_F32, D, 1>;
+    case 2: return paged_decode_merge<MIP_F32, D, 2>;
+    case 3: return paged_decode_merge<MIP_F32, D, 3>;
+    case 4: return paged_decode_merge<MIP_F32, D, 4>;
+    case 5: return paged_decode_merge<MIP_F32, D, 5>;
+    case 6: return paged_decode_merge<MIP_F32, D, 6>;
+    case 7: return paged_decode_merge<MIP_F32, D, 7>;
+    case 8: return paged_decode_merge<MIP_F32, D, 8>;
+    case 9: return paged_decode_merge<MIP_F32, D, 9>;
+    case 10: return paged_decode_merge<MIP_F32, D, 10>;
+    case 11: return paged_decode_merge<MIP_F32, D, 11>;
+    case 12: return paged_decode_merge<MIP_F32, D, 12>;
+    case 13: return paged_decode_merge<MIP_F32, D, 13>;
+    case 14: return paged_decode_merge<MIP_F32, D, 14>;
+    case 15: return paged_decode_merge<MIP_F32, D, 15>;
+    case 16: return paged_decode_merge<MIP_F32, D, 16>;
+    default: return nullptr;
+  }
+}
+
 KernelPair pick_kernel(Algo algo, int dtype, int d, int g) {
+  if (algo == Algo::kF32) return {f32_decode_kernel(d), d == 64 ? pick_f32_merge<64>(g) : pick_f32_merge<128>(g)};
   if (algo == Algo::kMfma) {
     switch (dtype) {
       case MIP_F16: return pick_mfma_d<MIP_F16>(d, g);
@@ -918,6 +946,8 @@ int valu_prefill_launch(void* out, int64_t out_stride_tok, int64_t out_stride_he
   a.max_q_len = max_q_len;
   a.gsplit = vsplit;
   a.group = group;
+  if (f32_eligible(dtype, head_dim, group) && static_cast<int64_t>(max_q_len) * group < (int64_t{1} << 30))
+    return f32_prefill_launch(a, num_seqs, head_dim, stream);
   hipLaunchKernelGGL(kp.part, dim3(static_cast<unsigned>(grid_x), num_kv_heads * vsplit, 1), dim3(kNW * kWave), 0,
                      stream, a);
   return status_from_hip(hipGetLastError());
@@ -970,7 +1000,8 @@ int paged_decode_impl(void* out, int64_t out_stride_b, int64_t out_stride_h, con
   if (!kp.part) return MIP_EUNSUPPORTED;
   const int64_t es = dtype == MIP_F32 ? 4 : 2;
   if ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15) return MIP_EINVAL;
-  const uint64_t q_align = wl.algo == Algo::kValu ? 3 : 15;  // MFMA kernels read q rows with 16-byte loads
+  // The 16-bit MFMA kernels read q rows with 16-byte loads.
+  const uint64_t q_align = wl.algo == Algo::kValu || wl.algo == Algo::kF32 ? 3 : 15;
   if ((reinterpret_cast<uintptr_t>(q) | static_cast<uint64_t>(q_stride_b * es) |
        static_cast<uint64_t>(q_stride_h * es)) & q_align)
     return MIP_EINVAL;

@@ -305,6 +305,18 @@ int mip_paged_prefill(void* out, int64_t out_stride_tok, int64_t out_stride_head
                       int32_t head_dim, int32_t block_size, int32_t max_blocks_per_seq, float scale,
                       int32_t dtype, void* stream);
 
+/*
+ * Index arrays of a packed prefill step (engine/kv_cache.py:230-250, 562-573), from the tensors
+ * mip_paged_prefill takes: for new token i of sequence s, packed row r = cu_q[s] + i,
+ *     positions[r]    = p = ctx_start[s] + i
+ *     slot_mapping[r] = block_tables[s][p / block_size] * block_size + p % block_size
+ * and last_index[s] = cu_q[s + 1] - 1. max_q_len must be >= every cu_q[s + 1] - cu_q[s], and
+ * every position must lie in its sequence's table.
+ */
+int mip_prefill_index(int64_t* positions, int64_t* slot_mapping, int64_t* last_index, const int32_t* cu_q,
+                      const int32_t* ctx_start, const int32_t* block_tables, int64_t bt_stride,
+                      int32_t num_seqs, int32_t max_q_len, int32_t block_size, void* stream);
+
 /* Workspace bytes mip_paged_decode and mip_paged_decode_append need for this shape (0 when
  * they need none). */
 size_t mip_paged_decode_workspace(int32_t batch, int32_t num_heads, int32_t num_kv_heads,

@@ -32,6 +32,7 @@ EXPORTED = (
     "mip_paged_prefill",
     "mip_copy_blocks",
     "mip_copy_blocks_host",
+    "mip_prefill_index",
     "mip_add_rms_norm",
     "mip_silu_mul",
     "mip_norm_linear",
@@ -85,6 +86,7 @@ _SIGNATURES = {
         [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _vp, _vp,
          _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _vp],
     ),
+    "mip_prefill_index": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp]),
     "mip_copy_blocks": (_c.c_int, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp]),
     "mip_copy_blocks_host": (_c.c_int, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp]),
     "mip_add_rms_norm": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _f32, _i32, _vp]),

@@ -22,6 +22,7 @@ from __future__ import annotations
 
 from collections import OrderedDict
 from collections.abc import Sequence
+from itertools import chain
 
 import numpy as np
 import torch
@@ -495,38 +496,55 @@ class PackedPrefillContext:
         self.cache = cache
         self.slots = list(slots)
         self.lengths = list(lengths)
+        if not self.slots:
+            raise ValueError("a packed prefill needs at least one sequence")
         self.starts = [cache.lengths[s] for s in self.slots]
         for s, start, n in zip(self.slots, self.starts, self.lengths):
             if not cache.ensure_capacity(s, start + n):
                 raise ValueError(f"no room in the KV cache for {start + n} tokens")
         cache.prepare_writes(self.slots, self.starts, self.lengths)
         dev = cache.k.device
-        self.positions = torch.from_numpy(np.concatenate(
-            [np.arange(a, a + n, dtype=np.int64) for a, n in zip(self.starts, self.lengths)])).to(dev)
-        blocks, offsets = cache._write_index_np(self.slots, self.starts, self.lengths)
-        both = torch.from_numpy(np.concatenate([blocks, offsets, blocks * cache.block_size + offsets])).to(dev)
-        n_tok = blocks.shape[0]
-        self.write_at = (both[:n_tok], both[n_tok:2 * n_tok])
-        self.slot_mapping = both[2 * n_tok:]
         self.has_prefix = any(self.starts)
         self.ends = [a + n for a, n in zip(self.starts, self.lengths)]
         # Inputs of the paged prefill kernel: packed row offsets, cached lengths, tables.
-        self.max_q_len = max(self.lengths) if self.lengths else 0
-        nb = max(1, cache.blocks_for(max(self.ends))) if self.ends else 1
-        tables = np.zeros((len(self.slots), nb), dtype=np.int32)
-        for i, s in enumerate(self.slots):
-            row = cache.block_tables[s][:nb]
-            tables[i, :len(row)] = row
-        cu = np.zeros(len(self.slots) + 1, dtype=np.int32)
-        cu[1:] = np.cumsum(self.lengths)
-        i32 = torch.from_numpy(np.concatenate([cu, np.asarray(self.starts, dtype=np.int32), tables.reshape(-1)])).to(dev)
+        self.max_q_len = max(self.lengths)
+        nb = max(1, cache.blocks_for(max(self.ends)))
         s_n = len(self.slots)
-        self.cu_q, self.ctx_start = i32[:s_n + 1], i32[s_n + 1:2 * s_n + 1]
-        self.block_tables = i32[2 * s_n + 1:].view(s_n, nb)
+        host = torch.empty(2 * s_n + 1 + s_n * nb, dtype=torch.int32, pin_memory=dev.type == "cuda")
+        i32 = host.numpy()
+        i32[0] = 0
+        np.cumsum(self.lengths, out=i32[1:s_n + 1])
+        i32[s_n + 1:2 * s_n + 1] = self.starts
+        rows = [cache.block_tables[s][:nb] for s in self.slots]
+        widths = np.fromiter(map(len, rows), dtype=np.int64, count=s_n)
+        tables = i32[2 * s_n + 1:].reshape(s_n, nb)
+        tables.fill(0)
+        tables[np.arange(nb) < widths[:, None]] = np.fromiter(chain.from_iterable(rows), dtype=np.int32,
+                                                              count=int(widths.sum()))
+        n_tok = int(i32[s_n])
+        on_dev = host.to(dev, non_blocking=True)
+        self.cu_q, self.ctx_start = on_dev[:s_n + 1], on_dev[s_n + 1:2 * s_n + 1]
+        self.block_tables = on_dev[2 * s_n + 1:].view(s_n, nb)
+        if dev.type == "cuda":
+            # Positions and slots of the new tokens, made where the tables are. Everything is in
+            # place when the constructor returns, on whatever stream it is used then.
+            self.positions, self.slot_mapping, self.last_index = paged_ops.prefill_index(
+                self.cu_q, self.ctx_start, self.block_tables, n_tok, self.max_q_len, cache.block_size)
+            torch.cuda.current_stream(dev).synchronize()
+        else:
+            self.positions = torch.from_numpy(np.concatenate(
+                [np.arange(a, a + n, dtype=np.int64) for a, n in zip(self.starts, self.lengths)]))
+            self.slot_mapping = cache.slot_mapping(self.slots, self.starts, self.lengths)
+            self.last_index = torch.tensor(self.lengths).cumsum(0) - 1
         self._mask_built = False
         self._mask = None
         self._read_at = None
-        self.last_index = torch.tensor(self.lengths, device=dev).cumsum(0) - 1
+
+    @property
+    def write_at(self) -> tuple[torch.Tensor, torch.Tensor]:
+        """``(block, offset)`` of each new token (engine/kv_cache.py:247), from ``slot_mapping``."""
+        bs = self.cache.block_size
+        return torch.div(self.slot_mapping, bs, rounding_mode="floor"), self.slot_mapping % bs
 
     def _build_mask(self) -> None:
         """The reference's mask and read-back index (engine/kv_cache.py:262-279), built on demand."""

@@ -432,6 +432,25 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
     return out
 
 
+def prefill_index(cu_q: torch.Tensor, ctx_start: torch.Tensor, block_tables: torch.Tensor, n_tokens: int,
+                  max_q_len: int, block_size: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """``positions`` and ``slot_mapping`` (int64 ``[n_tokens]``) of a packed prefill step's new tokens, and
+    ``last_index`` (int64 ``[S]``), from the tensors :func:`paged_prefill` takes. Follows
+    engine/kv_cache.py:230-250, 562-573.
+    """
+    _require_device(cu_q, ctx_start, block_tables)
+    s = ctx_start.shape[0]
+    out = torch.empty(2 * n_tokens + s, dtype=torch.int64, device=cu_q.device)
+    positions, slots, last = out[:n_tokens], out[n_tokens:2 * n_tokens], out[2 * n_tokens:]
+    if s:
+        st = _native.load().mip_prefill_index(positions.data_ptr(), slots.data_ptr(), last.data_ptr(), cu_q.data_ptr(),
+                                              ctx_start.data_ptr(), block_tables.data_ptr(), block_tables.stride(0), s,
+                                              max_q_len, block_size, _stream_ptr(cu_q.device))
+        if st:
+            _native.check(st, "mip_prefill_index")
+    return positions, slots, last
+
+
 def prepare_paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor,
                           cu_q: torch.Tensor, ctx_start: torch.Tensor, max_q_len: int, scale: float | None = None,
                           out: torch.Tensor | None = None, max_blocks: int | None = None):

@@ -393,6 +393,61 @@ int mip_norm_linear(void* out, const void* x, const void* norm, float eps, const
 int mip_linear_residual(void* out, const void* a, const void* weight, const void* residual, int32_t m,
                         int32_t n, int32_t k, int32_t dtype, void* stream);
 
+/*
+ * The layer calls of one step. Every layer of a step passes the same sequences, strides and sizes
+ * and other tensors of the same layout; these entry points take what stays the same as a host
+ * struct (read during the call, owned by the caller) and the layer's pointers as arguments. Each is
+ * the call named beside it, with that call's checks and results. Fields are that call's arguments.
+ */
+typedef struct mip_decode_step {
+  int64_t k_stride_tok, k_stride_head, v_stride_tok, v_stride_head; /* append only */
+  const int64_t* slot_mapping;                                      /* append only */
+  int64_t out_stride_b, out_stride_h, q_stride_b, q_stride_h, num_cache_blocks;
+  const int32_t* block_tables;
+  int64_t bt_stride;
+  const int32_t* context_lens;
+  void* workspace;
+  size_t workspace_bytes;
+  const void* plan;
+  size_t plan_bytes;
+  int32_t batch, num_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, dtype;
+  float scale;
+} mip_decode_step;
+
+typedef struct mip_rope_step {
+  int64_t q_stride_tok, q_stride_head, k_stride_tok, k_stride_head, v_stride_tok, v_stride_head, cs_stride_tok;
+  int64_t num_cache_blocks;
+  const int64_t* slot_mapping;
+  int32_t n_tokens, num_heads, num_kv_heads, head_dim, block_size, dtype;
+} mip_rope_step;
+
+typedef struct mip_prefill_step {
+  int64_t k_stride_tok, k_stride_head, v_stride_tok, v_stride_head; /* append only */
+  const int64_t* slot_mapping;                                      /* append only */
+  int64_t out_stride_tok, out_stride_head, q_stride_tok, q_stride_head, num_cache_blocks;
+  const int32_t* block_tables;
+  int64_t bt_stride;
+  const int32_t* cu_q;
+  const int32_t* ctx_start;
+  int32_t n_tokens, num_seqs, max_q_len, num_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, dtype;
+  float scale;
+} mip_prefill_step;
+
+/* mip_paged_decode_append */
+int mip_decode_step_append(const mip_decode_step* step, const void* k_new, const void* v_new, void* out,
+                           const void* q, void* k_cache, void* v_cache, void* stream);
+/* mip_paged_decode */
+int mip_decode_step_attend(const mip_decode_step* step, void* out, const void* q, const void* k_cache,
+                           const void* v_cache, void* stream);
+/* mip_rope_kv_append */
+int mip_rope_step_append(const mip_rope_step* step, void* q, void* k, const void* v, const void* cos,
+                         const void* sin, void* k_cache, void* v_cache, void* stream);
+/* mip_kv_append of the packed new tokens, and mip_paged_prefill */
+int mip_prefill_step_append(const mip_prefill_step* step, const void* k_new, const void* v_new, void* k_cache,
+                            void* v_cache, void* stream);
+int mip_prefill_step_attend(const mip_prefill_step* step, void* out, const void* q, const void* k_cache,
+                            const void* v_cache, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

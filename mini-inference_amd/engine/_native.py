@@ -33,6 +33,11 @@ EXPORTED = (
     "mip_copy_blocks",
     "mip_copy_blocks_host",
     "mip_prefill_index",
+    "mip_decode_step_append",
+    "mip_decode_step_attend",
+    "mip_rope_step_append",
+    "mip_prefill_step_append",
+    "mip_prefill_step_attend",
     "mip_add_rms_norm",
     "mip_silu_mul",
     "mip_norm_linear",
@@ -44,6 +49,38 @@ PROBE_EXPORTED = ("mip_hbm_read_probe",)
 
 _c = ctypes
 _i32, _i64, _sz, _vp, _f32 = _c.c_int32, _c.c_int64, _c.c_size_t, _c.c_void_p, _c.c_float
+
+
+class DecodeStep(_c.Structure):
+    """``mip_decode_step``: what every layer's decode call of one step shares."""
+
+    _fields_ = [(n, _i64) for n in ("k_stride_tok", "k_stride_head", "v_stride_tok", "v_stride_head")] + [
+        ("slot_mapping", _vp)] + [(n, _i64) for n in ("out_stride_b", "out_stride_h", "q_stride_b", "q_stride_h",
+                                                      "num_cache_blocks")] + [
+        ("block_tables", _vp), ("bt_stride", _i64), ("context_lens", _vp), ("workspace", _vp), ("workspace_bytes", _sz),
+        ("plan", _vp), ("plan_bytes", _sz)] + [
+        (n, _i32) for n in ("batch", "num_heads", "num_kv_heads", "head_dim", "block_size", "max_blocks_per_seq",
+                            "dtype")] + [("scale", _f32)]
+
+
+class RopeStep(_c.Structure):
+    """``mip_rope_step``: what every layer's rotary embedding + append call of one step shares."""
+
+    _fields_ = [(n, _i64) for n in ("q_stride_tok", "q_stride_head", "k_stride_tok", "k_stride_head", "v_stride_tok",
+                                    "v_stride_head", "cs_stride_tok", "num_cache_blocks")] + [("slot_mapping", _vp)] + [
+        (n, _i32) for n in ("n_tokens", "num_heads", "num_kv_heads", "head_dim", "block_size", "dtype")]
+
+
+class PrefillStep(_c.Structure):
+    """``mip_prefill_step``: what every layer's packed prefill calls of one step share."""
+
+    _fields_ = [(n, _i64) for n in ("k_stride_tok", "k_stride_head", "v_stride_tok", "v_stride_head")] + [
+        ("slot_mapping", _vp)] + [(n, _i64) for n in ("out_stride_tok", "out_stride_head", "q_stride_tok",
+                                                      "q_stride_head", "num_cache_blocks")] + [
+        ("block_tables", _vp), ("bt_stride", _i64), ("cu_q", _vp), ("ctx_start", _vp)] + [
+        (n, _i32) for n in ("n_tokens", "num_seqs", "max_q_len", "num_heads", "num_kv_heads", "head_dim", "block_size",
+                            "max_blocks_per_seq", "dtype")] + [("scale", _f32)]
+
 
 _SIGNATURES = {
     "mip_version": (_c.c_int, []),
@@ -86,6 +123,11 @@ _SIGNATURES = {
         [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _vp, _vp,
          _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _vp],
     ),
+    "mip_decode_step_append": (_c.c_int, [_vp] * 8),
+    "mip_decode_step_attend": (_c.c_int, [_vp] * 6),
+    "mip_rope_step_append": (_c.c_int, [_vp] * 9),
+    "mip_prefill_step_append": (_c.c_int, [_vp] * 6),
+    "mip_prefill_step_attend": (_c.c_int, [_vp] * 6),
     "mip_prefill_index": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp]),
     "mip_copy_blocks": (_c.c_int, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp]),
     "mip_copy_blocks_host": (_c.c_int, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp]),

@@ -23,6 +23,7 @@ from __future__ import annotations
 from collections import OrderedDict
 from collections.abc import Sequence
 from itertools import chain
+from operator import ge
 
 import numpy as np
 import torch
@@ -216,14 +217,19 @@ class PagedKVCache:
         Returns the ``(src, dst)`` pairs copied. Raises if the pool cannot supply them.
         """
         pairs: list[tuple[int, int]] = []
+        bs, refs, tables = self.block_size, self._ref_counts, self.block_tables
         for slot, start, n in zip(slots, starts, counts):
             if n <= 0:
                 continue
-            table = self.block_tables[slot]
-            last = min((start + n - 1) // self.block_size, len(table) - 1)
-            for i in range(start // self.block_size, last + 1):
+            table = tables[slot]
+            first = start // bs
+            last = (start + n - 1) // bs
+            if first == last < len(table) and refs[table[first]] <= 1:
+                continue  # one block, already private: the usual decode write
+            last = min(last, len(table) - 1)
+            for i in range(first, last + 1):
                 old = table[i]
-                if self._ref_counts[old] > 1:
+                if refs[old] > 1:
                     if not self._free_blocks:
                         raise RuntimeError("not enough free KV cache blocks for copy-on-write")
                     new = self._new_block()
@@ -377,13 +383,16 @@ class PagedDecodeContext:
         self.cache = cache
         self.slots = list(slots)
         bs = cache.block_size
-        pos = [cache.lengths[s] for s in self.slots]
-        if any(p // bs >= len(cache.block_tables[s]) for p, s in zip(pos, self.slots)):
+        lengths, tables = cache.lengths, cache.block_tables
+        pos = [lengths[s] for s in self.slots]
+        at = [p // bs for p in pos]
+        rows = [tables[s] for s in self.slots]
+        if any(map(ge, at, map(len, rows))):
             raise ValueError("a sequence has no block for its next token (call ensure_capacity first)")
         cache.prepare_writes(self.slots, pos, [1] * len(self.slots))  # copy-on-write of shared blocks
         dt = cache.enable_device_tables()
         b = len(self.slots)
-        write_blocks = [cache.block_tables[s][p // bs] for s, p in zip(self.slots, pos)]
+        write_blocks = [row[i] for row, i in zip(rows, at)]
         flat, blocks = dt.flat_entries(cache.drain_journal())
         m = len(flat)
         # One int64 upload: slot ids | positions | slots | journal (flat index, block) | context
@@ -458,8 +467,7 @@ class PagedDecodeContext:
 
     def attend(self, layer_idx: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         """Append this step's k/v and attend (engine/kv_cache.py:611-620) in one fused call."""
-        k_layer, v_layer = self.cache.k[layer_idx], self.cache.v[layer_idx]
-        return self.calls.decode_append(q[:, :, 0], k[:, :, 0], v[:, :, 0], k_layer, v_layer).unsqueeze(2)
+        return self.calls.append_attend(layer_idx, q, k, v, self.cache.k, self.cache.v)
 
     def attend_rope(self, layer_idx: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor,
                     sin: torch.Tensor) -> torch.Tensor:
@@ -469,10 +477,9 @@ class PagedDecodeContext:
         decode kernel then reads every key, the new one included, from the pool. ``cos`` and
         ``sin`` are the ``[B, 1, 1, D]`` tables of the step.
         """
-        k_layer, v_layer = self.cache.k[layer_idx], self.cache.v[layer_idx]
-        q1 = q[:, :, 0]
-        self.calls.rope_append(q1, k[:, :, 0], v[:, :, 0], cos[:, 0, 0], sin[:, 0, 0], k_layer, v_layer)
-        return self.calls.decode(q1, k_layer, v_layer).unsqueeze(2)
+        calls, c = self.calls, self.cache
+        calls.rope_append(layer_idx, q, k, v, cos, sin, c.k, c.v)
+        return calls.attend(layer_idx, q, c.k, c.v)
 
     def commit(self) -> None:
         for s in self.slots:
@@ -539,6 +546,7 @@ class PackedPrefillContext:
         self._mask_built = False
         self._mask = None
         self._read_at = None
+        self._calls: paged_ops.PrefillStepCalls | None = None
 
     @property
     def write_at(self) -> tuple[torch.Tensor, torch.Tensor]:
@@ -577,11 +585,18 @@ class PackedPrefillContext:
             self._build_mask()
         return self._read_at
 
+    @property
+    def calls(self) -> paged_ops.PrefillStepCalls:
+        """The step's layer calls: the shared arguments are checked on the first layer only."""
+        if self._calls is None:
+            self._calls = paged_ops.PrefillStepCalls(self.block_tables, self.cu_q, self.ctx_start, self.slot_mapping,
+                                                     self.max_q_len, 1.0 / (self.cache.head_dim ** 0.5))
+        return self._calls
+
     def attend(self, layer_idx: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
-        k_layer, v_layer = self.cache.k[layer_idx], self.cache.v[layer_idx]
-        # k[0] is [Hkv, N, D]; the append kernel takes [N, Hkv, D] views with any strides.
-        paged_ops.kv_append(k_layer, v_layer, k[0].transpose(0, 1), v[0].transpose(0, 1), self.slot_mapping)
-        return self._attention(k_layer, v_layer, q, k, v)
+        calls, c = self.calls, self.cache
+        calls.append(layer_idx, k, v, c.k, c.v)
+        return calls.attend(layer_idx, q, c.k, c.v)
 
     def attend_rope(self, layer_idx: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor,
                     sin: torch.Tensor) -> torch.Tensor:
@@ -590,16 +605,9 @@ class PackedPrefillContext:
         ``cos``/``sin`` are ``[1, 1, N, D]``; q and k are rotated in place, so the prefill
         attention below sees the same tensors as after ``apply_rope``.
         """
-        k_layer, v_layer = self.cache.k[layer_idx], self.cache.v[layer_idx]
-        paged_ops.rope_kv_append(q[0].transpose(0, 1), k[0].transpose(0, 1), v[0].transpose(0, 1), cos[0, 0],
-                                 sin[0, 0], k_layer, v_layer, self.slot_mapping)
-        return self._attention(k_layer, v_layer, q, k, v)
-
-    def _attention(self, k_layer, v_layer, q, k, v) -> torch.Tensor:
-        # q is [1, Hq, N, D]; the kernel takes the [N, Hq, D] view and returns [N, Hq, D].
-        out = paged_ops.paged_prefill(q[0].transpose(0, 1), k_layer, v_layer, self.block_tables, self.cu_q,
-                                      self.ctx_start, self.max_q_len, scale=1.0 / (self.cache.head_dim ** 0.5))
-        return out.transpose(0, 1).unsqueeze(0)
+        calls, c = self.calls, self.cache
+        calls.rope_append(layer_idx, q, k, v, cos, sin, c.k, c.v)
+        return calls.attend(layer_idx, q, c.k, c.v)
 
     def commit(self) -> None:
         for slot, start, n in zip(self.slots, self.starts, self.lengths):

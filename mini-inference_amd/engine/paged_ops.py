@@ -7,6 +7,7 @@ here computes on the CPU: tensors that are not on a ROCm device raise.
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import numpy as np
@@ -140,15 +141,11 @@ def prepare_rope_kv_append(q: torch.Tensor | None, k: torch.Tensor, v: torch.Ten
     lib = _native.load()
     hq = 0 if q is None else q.shape[1]
     qp, qs0, qs1 = (None, 0, 0) if q is None else (q.data_ptr(), q.stride(0), q.stride(1))
-    # Positions of the per-call addresses are _ROPE_SLOTS (q, k, v, cos, sin, k_cache, v_cache).
     args = (qp, qs0, qs1, k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(), v.stride(0), v.stride(1),
             cos.data_ptr(), sin.data_ptr(), cos.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), nb,
             slot_mapping.data_ptr(), n, hq, hkv, d, bs, dtype_code(dt), _stream_ptr(k_cache.device))
     return PreparedCall(lib.mip_rope_kv_append, args, "mip_rope_kv_append",
                         (q, k, v, cos, sin, k_cache, v_cache, slot_mapping))
-
-
-_ROPE_SLOTS = (0, 3, 6, 9, 10, 12, 13)
 
 
 def rope_kv_append(q: torch.Tensor | None, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
@@ -264,8 +261,6 @@ def prepare_paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
             raise ValueError(f"the plan was made for shape {made_for}, not this call's {want}")
     plan_ptr = plan.data_ptr() if plan is not None else None
     plan_bytes = plan.numel() * 4 if plan is not None else 0
-    # Positions of the per-call addresses are _DECODE_SLOTS (out, q, k_cache, v_cache), and
-    # _APPEND_SLOTS (k, v, out, q, k_cache, v_cache) in the fused tuple below.
     args = (out.data_ptr(), out.stride(0), out.stride(1), q.data_ptr(), q.stride(0), q.stride(1),
             k_cache.data_ptr(), v_cache.data_ptr(), nb, block_tables.data_ptr(), block_tables.stride(0),
             context_lens.data_ptr(), b, hq, hkv, d, bs, mb, scale, ws_ptr, ws_bytes, plan_ptr, plan_bytes, code,
@@ -288,87 +283,201 @@ def prepare_paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
     return PreparedCall(lib.mip_paged_decode_append, fused, "mip_paged_decode_append", keep + (k, v, slot_mapping)), out
 
 
-_DECODE_SLOTS = (0, 3, 6, 7)
-_APPEND_SLOTS = (0, 1, 7, 10, 13, 14)
-
-
 def _layout(t: torch.Tensor) -> tuple:
     return (t.shape, t.stride(), t.dtype, t.device)
 
 
-class DecodeStepCalls:
-    """The per-layer calls of one decode step, with the step's fixed arguments checked once.
+class _LayerCalls:
+    """The per-layer calls of one step, with what the layers share checked and laid out once.
 
-    Within a step every layer's call takes the same block tables, context lengths, slot
-    mapping, plan and workspace; only q, k, v, the layer's pool and the output change, and
-    they keep one layout. Each method runs the full checks of :func:`prepare_paged_decode` /
-    :func:`prepare_rope_kv_append` when the layout of its tensors (shapes, strides, dtypes,
-    devices) differs from the call before, and otherwise issues the same C-ABI call with
-    the new addresses and the current stream. ``plan`` maps (num_heads, dtype) to the step's
-    work plan (or None).
+    Within a step every layer's call takes the same tables, lengths, slots and sizes; only the
+    layer's tensors change, and they keep one layout. The first call of a kind runs the full checks
+    (the ``prepare_*`` functions) and keeps their arguments as a struct of the C ABI; a later call
+    whose tensors have the same layout (shapes, strides, dtypes, devices) passes that struct, the
+    new addresses and the current stream. Any other call is checked in full again.
+
+    Tensors come as an attention layer has them, ``[B, H, T, D]``, and pools whole,
+    ``[L, num_blocks + 1, Hkv, block_size, D]``.
     """
+
+    def __init__(self) -> None:
+        # kind -> (layout key, address of the struct, layers, K and V layer bytes, the struct, kept tensors)
+        self._cached: dict[str, tuple] = {}
+
+    def _hit(self, kind: str, key: tuple, layer) -> tuple | None:
+        hit = self._cached.get(kind)
+        if hit is None or hit[0] != key or type(layer) is not int or not 0 <= layer < hit[2]:
+            return None
+        return hit
+
+    def _keep(self, kind: str, key: tuple, step, k_pool: torch.Tensor, v_pool: torch.Tensor, keep: tuple) -> None:
+        self._cached[kind] = (key, ctypes.addressof(step), k_pool.shape[0], k_pool.stride(0) * k_pool.element_size(),
+                              v_pool.stride(0) * v_pool.element_size(), step, keep)
+
+
+class DecodeStepCalls(_LayerCalls):
+    """The layer calls of one decode step (one token per sequence). ``plan`` maps (num_heads, dtype) to the
+    step's work plan (or None)."""
 
     def __init__(self, block_tables: torch.Tensor, context_lens: torch.Tensor, slot_mapping: torch.Tensor,
                  scale: float, max_blocks: int, plan) -> None:
+        super().__init__()
         self.block_tables, self.context_lens, self.slot_mapping = block_tables, context_lens, slot_mapping
         self.scale, self.max_blocks, self._plan = scale, max_blocks, plan
-        self._cached: dict[str, tuple] = {}  # kind -> (layout key, fn, argument list, kept tensors)
 
-    def _issue(self, kind: str, key: tuple, prepare, ptrs: tuple, slots: tuple, device: torch.device) -> None:
-        hit = self._cached.get(kind)
-        if hit is None or hit[0] != key:
-            call = prepare()
-            if call is _noop:
-                return
-            self._cached[kind] = (key, call._fn, list(call._args), call.keep)
-            call()
+    def append_attend(self, layer: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_pool: torch.Tensor,
+                      v_pool: torch.Tensor) -> torch.Tensor:
+        """:func:`paged_decode_append` of one layer; returns ``[B, Hq, 1, D]``."""
+        key = (_layout(q), _layout(k), _layout(v), _layout(k_pool), _layout(v_pool))
+        hit = self._hit("append", key, layer)
+        if hit is not None:
+            _, step, _, kb, vb, _, _ = hit
+            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+            st = _native.load().mip_decode_step_append(step, k.data_ptr(), v.data_ptr(), out.data_ptr(), q.data_ptr(),
+                                                       k_pool.data_ptr() + layer * kb, v_pool.data_ptr() + layer * vb,
+                                                       _stream_ptr(q.device))
+            if st:
+                _native.check(st, "mip_decode_step_append")
+            return out
+        q1 = q[:, :, 0]
+        call, out = prepare_paged_decode(q1, k_pool[layer], v_pool[layer], self.block_tables, self.context_lens,
+                                         self.scale, None, self.max_blocks, append=(k[:, :, 0], v[:, :, 0],
+                                                                                    self.slot_mapping),
+                                         plan=self._plan(q1.shape[1], q1.dtype))
+        call()
+        if call is not _noop and q.shape[2] == k.shape[2] == v.shape[2] == 1:
+            a = call._args
+            self._keep("append", key, self._struct(a[7:], a[2:6], a[6]), k_pool, v_pool, call.keep)
+        return out.unsqueeze(2)
+
+    def attend(self, layer: int, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor) -> torch.Tensor:
+        """:func:`paged_decode` of one layer; returns ``[B, Hq, 1, D]``."""
+        key = (_layout(q), _layout(k_pool), _layout(v_pool))
+        hit = self._hit("decode", key, layer)
+        if hit is not None:
+            _, step, _, kb, vb, _, _ = hit
+            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+            st = _native.load().mip_decode_step_attend(step, out.data_ptr(), q.data_ptr(),
+                                                       k_pool.data_ptr() + layer * kb, v_pool.data_ptr() + layer * vb,
+                                                       _stream_ptr(q.device))
+            if st:
+                _native.check(st, "mip_decode_step_attend")
+            return out
+        q1 = q[:, :, 0]
+        call, out = prepare_paged_decode(q1, k_pool[layer], v_pool[layer], self.block_tables, self.context_lens,
+                                         self.scale, None, self.max_blocks, plan=self._plan(q1.shape[1], q1.dtype))
+        call()
+        if call is not _noop and q.shape[2] == 1:
+            self._keep("decode", key, self._struct(call._args, (0, 0, 0, 0), None), k_pool, v_pool, call.keep)
+        return out.unsqueeze(2)
+
+    @staticmethod
+    def _struct(a: tuple, kv_strides: tuple, slots) -> _native.DecodeStep:
+        # a: the arguments of mip_paged_decode
+        return _native.DecodeStep(*kv_strides, slots, a[1], a[2], a[4], a[5], a[8], a[9], a[10], a[11], a[19], a[20],
+                                  a[21], a[22], *a[12:18], a[23], a[18])
+
+    def rope_append(self, layer: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor,
+                    sin: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor) -> None:
+        """:func:`rope_kv_append` of one layer (q and k rotated in place); cos, sin ``[B, 1, 1, D]``."""
+        key = (_layout(q), _layout(k), _layout(v), _layout(cos), _layout(sin), _layout(k_pool), _layout(v_pool))
+        if _rope_hit(self, layer, key, q, k, v, cos, sin, k_pool, v_pool):
             return
-        _, fn, args, _ = hit
-        for i, p in zip(slots, ptrs):
-            args[i] = p
-        args[-1] = _stream_ptr(device)
-        st = fn(*args)
-        if st:
-            _native.check(st, fn.__name__)
+        call = prepare_rope_kv_append(q[:, :, 0], k[:, :, 0], v[:, :, 0], cos[:, 0, 0], sin[:, 0, 0], k_pool[layer],
+                                      v_pool[layer], self.slot_mapping)
+        call()
+        if call is not _noop and all(t.shape[2] == 1 for t in (q, k, v)):
+            self._keep("rope", key, _rope_struct(call._args), k_pool, v_pool, call.keep)
 
-    def decode_append(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
-                      v_cache: torch.Tensor) -> torch.Tensor:
-        """:func:`paged_decode_append` of one layer; returns ``out [B, Hq, D]``."""
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        key = (_layout(q), _layout(k), _layout(v), _layout(k_cache), _layout(v_cache))
 
-        def prepare():
-            return prepare_paged_decode(q, k_cache, v_cache, self.block_tables, self.context_lens, self.scale, out,
-                                        self.max_blocks, append=(k, v, self.slot_mapping),
-                                        plan=self._plan(q.shape[1], q.dtype))[0]
+def _rope_hit(calls: _LayerCalls, layer, key, q, k, v, cos, sin, k_pool, v_pool) -> bool:
+    hit = calls._hit("rope", key, layer)
+    if hit is None:
+        return False
+    _, step, _, kb, vb, _, _ = hit
+    st = _native.load().mip_rope_step_append(step, q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(),
+                                             sin.data_ptr(), k_pool.data_ptr() + layer * kb,
+                                             v_pool.data_ptr() + layer * vb, _stream_ptr(k.device))
+    if st:
+        _native.check(st, "mip_rope_step_append")
+    return True
 
-        self._issue("append", key, prepare, (k.data_ptr(), v.data_ptr(), out.data_ptr(), q.data_ptr(),
-                                             k_cache.data_ptr(), v_cache.data_ptr()), _APPEND_SLOTS, q.device)
-        return out
 
-    def decode(self, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor) -> torch.Tensor:
-        """:func:`paged_decode` of one layer; returns ``out [B, Hq, D]``."""
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        key = (_layout(q), _layout(k_cache), _layout(v_cache))
+def _rope_struct(a: tuple) -> _native.RopeStep:
+    # a: the arguments of mip_rope_kv_append
+    return _native.RopeStep(a[1], a[2], a[4], a[5], a[7], a[8], a[11], a[14], a[15], *a[16:22])
 
-        def prepare():
-            return prepare_paged_decode(q, k_cache, v_cache, self.block_tables, self.context_lens, self.scale, out,
-                                        self.max_blocks, plan=self._plan(q.shape[1], q.dtype))[0]
 
-        self._issue("decode", key, prepare, (out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr()),
-                    _DECODE_SLOTS, q.device)
-        return out
+class PrefillStepCalls(_LayerCalls):
+    """The layer calls of one packed prefill step; q, k, v ``[1, H, N, D]``, cos and sin ``[1, 1, N, D]``."""
 
-    def rope_append(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                    k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
-        """:func:`rope_kv_append` of one layer (q and k rotated in place)."""
-        key = (_layout(q), _layout(k), _layout(v), _layout(cos), _layout(sin), _layout(k_cache), _layout(v_cache))
+    def __init__(self, block_tables: torch.Tensor, cu_q: torch.Tensor, ctx_start: torch.Tensor,
+                 slot_mapping: torch.Tensor, max_q_len: int, scale: float) -> None:
+        super().__init__()
+        self.block_tables, self.cu_q, self.ctx_start, self.slot_mapping = block_tables, cu_q, ctx_start, slot_mapping
+        self.max_q_len, self.scale = max_q_len, scale
 
-        def prepare():
-            return prepare_rope_kv_append(q, k, v, cos, sin, k_cache, v_cache, self.slot_mapping)
+    def append(self, layer: int, k: torch.Tensor, v: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor) -> None:
+        """:func:`kv_append` of one layer's new tokens."""
+        key = (_layout(k), _layout(v), _layout(k_pool), _layout(v_pool))
+        hit = self._hit("append", key, layer)
+        if hit is not None:
+            _, step, _, kb, vb, _, _ = hit
+            st = _native.load().mip_prefill_step_append(step, k.data_ptr(), v.data_ptr(), k_pool.data_ptr() + layer * kb,
+                                                        v_pool.data_ptr() + layer * vb, _stream_ptr(k_pool.device))
+            if st:
+                _native.check(st, "mip_prefill_step_append")
+            return
+        # k[0] is [Hkv, N, D]; the append kernel takes [N, Hkv, D] views with any strides.
+        call = prepare_kv_append(k_pool[layer], v_pool[layer], k[0].transpose(0, 1), v[0].transpose(0, 1),
+                                 self.slot_mapping)
+        call()
+        if call is not _noop and k.shape[0] == v.shape[0] == 1:
+            a = call._args
+            step = _native.PrefillStep(k_stride_tok=a[2], k_stride_head=a[3], v_stride_tok=a[4], v_stride_head=a[5],
+                                       slot_mapping=a[9], num_cache_blocks=a[8], n_tokens=a[10], num_kv_heads=a[11],
+                                       head_dim=a[12], block_size=a[13], dtype=a[14])
+            self._keep("append", key, step, k_pool, v_pool, call.keep)
 
-        self._issue("rope", key, prepare, (q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-                                           k_cache.data_ptr(), v_cache.data_ptr()), _ROPE_SLOTS, k.device)
+    def rope_append(self, layer: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor,
+                    sin: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor) -> None:
+        """:func:`rope_kv_append` of one layer's new tokens (q and k rotated in place)."""
+        key = (_layout(q), _layout(k), _layout(v), _layout(cos), _layout(sin), _layout(k_pool), _layout(v_pool))
+        if _rope_hit(self, layer, key, q, k, v, cos, sin, k_pool, v_pool):
+            return
+        call = prepare_rope_kv_append(q[0].transpose(0, 1), k[0].transpose(0, 1), v[0].transpose(0, 1), cos[0, 0],
+                                      sin[0, 0], k_pool[layer], v_pool[layer], self.slot_mapping)
+        call()
+        if call is not _noop and all(t.shape[0] == 1 for t in (q, k, v)):
+            self._keep("rope", key, _rope_struct(call._args), k_pool, v_pool, call.keep)
+
+    def attend(self, layer: int, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor) -> torch.Tensor:
+        """:func:`paged_prefill` of one layer; returns ``[1, Hq, N, D]``, a view of ``[N, Hq, D]``."""
+        key = (_layout(q), _layout(k_pool), _layout(v_pool))
+        hit = self._hit("attend", key, layer)
+        if hit is not None:
+            _, step, _, kb, vb, _, _ = hit
+            _, hq, n, d = q.shape
+            out = torch.empty_strided((1, hq, n, d), (hq * d, d, hq * d, 1), dtype=q.dtype, device=q.device)
+            st = _native.load().mip_prefill_step_attend(step, out.data_ptr(), q.data_ptr(),
+                                                        k_pool.data_ptr() + layer * kb, v_pool.data_ptr() + layer * vb,
+                                                        _stream_ptr(q.device))
+            if st:
+                _native.check(st, "mip_prefill_step_attend")
+            return out
+        # q is [1, Hq, N, D]; the kernel takes the [N, Hq, D] view and returns [N, Hq, D].
+        call, out = prepare_paged_prefill(q[0].transpose(0, 1), k_pool[layer], v_pool[layer], self.block_tables,
+                                          self.cu_q, self.ctx_start, self.max_q_len, scale=self.scale)
+        call()
+        if q.shape[0] == 1 and q.shape[2] > 0:
+            a = call._args
+            step = _native.PrefillStep(out_stride_tok=a[1], out_stride_head=a[2], q_stride_tok=a[4], q_stride_head=a[5],
+                                       num_cache_blocks=a[8], block_tables=a[9], bt_stride=a[10], cu_q=a[11],
+                                       ctx_start=a[12], num_seqs=a[13], max_q_len=a[14], num_heads=a[15],
+                                       num_kv_heads=a[16], head_dim=a[17], block_size=a[18], max_blocks_per_seq=a[19],
+                                       scale=a[20], dtype=a[21])
+            self._keep("attend", key, step, k_pool, v_pool, call.keep)
+        return out.transpose(0, 1).unsqueeze(0)
 
 
 def prepare_decode_plan(context_lens: torch.Tensor, block_tables: torch.Tensor, num_heads: int, num_kv_heads: int,

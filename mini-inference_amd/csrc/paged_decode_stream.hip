@@ -1428,6 +1428,11 @@ constexpr int64_t kPartsSegments = 16;
 int stream_wide_merge(int64_t segments) { return segments <= kWideMergeSegments ? 1 : 0; }
 int stream_merge_parts(int64_t segments) { return segments <= kPartsSegments ? kStreamParts : 1; }
 
+// Most pieces a segment of n tiles can be cut into. W <= ceil(T / min_tiles) wavefronts share T
+// tiles, so with min_tiles >= 4 a range holds at least floor(T / ceil(T / 4)) >= 2 tiles from T = 3
+// on: a segment meets at most (n - 2) / 2 whole ranges and one partial range at each end.
+int64_t most_pieces(int64_t n, int min_tiles) { return min_tiles >= 4 ? n / 2 + 1 : n; }
+
 // Most pieces per segment on average (see stream_active_waves). With the one- or two-stream
 // merge, 64 measured best for one to four long sequences (one-stream merge, B=1 at 32k keys:
 // 74 -> 32 us per call; 128: 31 us, 256: 42 us, 32: 46 us; two-stream merge: 26.4 us, 128:
@@ -1533,7 +1538,11 @@ int stream_launch(const StreamConfig& cfg, const StreamArgs& sa_in, int dtype, i
                      sa.plan_tile_off, sa.plan_wave_cap, sa);
   const int64_t segments = static_cast<int64_t>(batch) * num_kv_heads;
   const int wide = stream_wide_merge(segments);
-  sa.parts = stream_merge_parts(segments);
+  // No segment reaches the length at which the merge starts to cut it into runs: one run, no fold
+  // (the same work split and sums; B=1 with short tables: 3 launches to 2, 9.6 -> 6.3 us of host
+  // time per layer and 1.5 us of GPU time).
+  const int64_t most_tiles = (static_cast<int64_t>(sa.a.max_blocks) * sa.a.bs + 15) / 16;
+  sa.parts = most_pieces(most_tiles, sa.min_tiles) <= kWideMergeStreams * kMergeChunk ? 1 : stream_merge_parts(segments);
   hipLaunchKernelGGL(p.merge[fused][planned][wide], dim3(num_kv_heads, batch, sa.parts),
                      dim3(wide ? 256 * kWideMergeStreams : 256), 0, stream, sa.plan, sa.plan_seg_off, num_kv_heads,
                      sa);

@@ -383,6 +383,10 @@ int mip_silu_mul(void* out, const void* gate_up, int32_t rows, int32_t inter, in
  * mip_norm_linear:     h   = rnd(norm * rnd(x * rsqrt(mean(x^2) + eps)))       [m][k]
  *                      out = rnd(h weight^T + bias)                            [m][n]  (bias may be NULL)
  *   with gate_up != 0: y   = rnd(h weight^T), out = rnd(rnd(silu(y[:, :n/2])) * y[:, n/2:])   [m][n/2]  (bias NULL)
+ * mip_qkv_linear:      mip_norm_linear's out (h = x where norm is NULL), its first rot_heads heads of
+ *                      head_dim columns then rotated as mip_rope_kv_append rotates q and k, with row
+ *                      r's cos and sin at cos / sin + r * cs_stride_tok (elements; 8-byte aligned rows).
+ *                      head_dim must be a multiple of 16 and divide n.
  * mip_linear_residual: out = rnd(residual + rnd(a weight^T))                   [m][n]; out may be residual
  *
  * n must be a multiple of 16 and k of 32, every address 16-byte aligned; other calls are
@@ -390,6 +394,9 @@ int mip_silu_mul(void* out, const void* gate_up, int32_t rows, int32_t inter, in
  */
 int mip_norm_linear(void* out, const void* x, const void* norm, float eps, const void* weight, const void* bias,
                     int32_t m, int32_t n, int32_t k, int32_t gate_up, int32_t dtype, void* stream);
+int mip_qkv_linear(void* out, const void* x, const void* norm, float eps, const void* weight, const void* bias,
+                   const void* cos, const void* sin, int64_t cs_stride_tok, int32_t m, int32_t n, int32_t k,
+                   int32_t head_dim, int32_t rot_heads, int32_t dtype, void* stream);
 int mip_linear_residual(void* out, const void* a, const void* weight, const void* residual, int32_t m,
                         int32_t n, int32_t k, int32_t dtype, void* stream);
 

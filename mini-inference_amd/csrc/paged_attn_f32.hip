@@ -100,7 +100,8 @@ __global__ __launch_bounds__(kNW * kWave) void paged_attn_f32(DecodeArgs a) {
   constexpr int T = D / 16;  // dim tiles
   __shared__ float sh_acc[kNW][kRows][D + 4];  // + 4: the 16 rows of a store spread over the banks
   __shared__ float sh_m[kNW][kRows], sh_l[kNW][kRows];
-  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, c = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & (kWave - 1), c = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int kvh = blockIdx.y;
 
   // The workgroup's rows: row r is query row q0 + r / group of q, head kvh * group + r % group,

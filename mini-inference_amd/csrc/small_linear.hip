@@ -1,6 +1,7 @@
 // Linear layers of a decode step (few rows), with the work around them fused in:
 //     y = A W^T                      A: the input rows, or their RMS norm computed on the fly
-//     out = y (+ bias)               or  residual + y,  or  silu(y[:, :I]) * y[:, I:]
+//     out = y (+ bias), its q and k heads rotated (rotary embedding) where asked,
+//           or  residual + y,  or  silu(y[:, :I]) * y[:, I:]
 //
 // Reference semantics: engine/model.py's qkv_proj(input_norm(x)), x + o_proj(..),
 // silu * up of gate_up_proj(post_attn_norm(x)), x + down_proj(..). Products accumulate in fp32;
@@ -24,7 +25,8 @@
 // separate kernels it takes the place of), 0.5B shapes at 8 rows: norm + qkv 4.5 against 8.6 us,
 // norm + gate + up + silu 9.3 / 14.6 (17.4 MB, 1.9 TB/s; a bare read of the weights in this split
 // takes 6.1), o + residual 3.8 / 8.5, down + residual 10.5 / 20.3; at 64 rows 5.7 / 11.2,
-// 16.3 / 18.3, 4.2 / 10.0, 12.0 / 19.1. With more rows every workgroup's reads of A (L2 to
+// 16.3 / 18.3, 4.2 / 10.0, 12.0 / 19.1. The rotation at the end of the q, k, v projection costs 0.7 us
+// and saves the 3.2 to 5 us kernel that rotates and appends (the decode's merge appends instead). With more rows every workgroup's reads of A (L2 to
 // registers) take over: gate + up 27 / 18 us at 65 rows, which is left to the library.
 #include "mip_common.h"
 
@@ -56,21 +58,34 @@ struct LinearArgs {
   const char* residual;  // [m, n] or null
   const char* norm;      // [k] or null
   char* out;             // [m, n] (silu: n / 2 columns)
+  const char* cos;       // rope: [m, head_dim] rows, cs_st bytes apart
+  const char* sin;
+  int64_t cs_st;
   int m, n, k, m_tiles, n_tiles;
+  int head_dim, rot_heads;  // rope: the first rot_heads heads of the n columns are rotated
   float eps, inv_k;
 };
 
-enum Epilogue { kPlain = 0, kResidual = 1, kSilu = 2 };
+enum Epilogue { kPlain = 0, kResidual = 1, kSilu = 2, kRope = 3 };
+
+// First column of rope tile n0 / 16: its head, and 8 columns of that head's first half.
+__device__ __forceinline__ int pair_column(int n0, int head_dim) {
+  const int head = n0 / head_dim;
+  return head * head_dim + ((n0 - head * head_dim) >> 1);
+}
 
 // Tiles of 16 x 16: TM over rows, TN over weight rows. A silu tile's 16 weight rows are 8 gate rows
-// and the 8 up rows of the same output columns, so its output is 8 wide.
+// and the 8 up rows of the same output columns, so its output is 8 wide; a rope tile's are 8 rows
+// of a head's first half and the 8 that rotate with them.
 template <int DT, int TM, int TN, int NW, int U, bool NORM, int EPI>
 __global__ __launch_bounds__(NW * 64) void small_linear_kernel(LinearArgs p) {
   using E = typename Mfma<DT>::E;
   constexpr int kCols = EPI == kSilu ? 8 : 16;  // output columns of a tile
   __shared__ f32x4 part[NW][TM * TN][64];
   __shared__ float sums[NORM ? NW : 1][TM * 16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // The wavefront's index as a scalar: the matrix instructions below stand under tests of its k-range,
+  // and they ignore the lane mask, so those tests have to be branches.
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = lane & 15, quad = lane >> 4;
 
   // Workgroup b: XCD b & 7 takes the column tiles congruent to it, every row tile of one in turn.
@@ -87,12 +102,42 @@ __global__ __launch_bounds__(NW * 64) void small_linear_kernel(LinearArgs p) {
   for (int j = 0; j < TN; ++j) {
     int r = n0 + j * kCols + row;
     if (EPI == kSilu && row >= 8) r += (p.n >> 1) - 8;
+    if (EPI == kRope) r = pair_column(n0 + j * 16, p.head_dim) + (row < 8 ? row : (p.head_dim >> 1) + row - 8);
     wp[j] = p.w + (static_cast<int64_t>(r) * p.k + quad * 8) * 2;
   }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int r = m0 + i * 16 + row;
     ap[i] = p.a + (static_cast<int64_t>(r < p.m ? r : p.m - 1) * p.k + quad * 8) * 2;
+  }
+  // What the epilogue adds, requested ahead of everything: output o = threadIdx.x (one each at most).
+  const int half = EPI == kRope ? p.head_dim >> 1 : 0;
+  constexpr int kLanes = 4 * kCols / (EPI == kRope ? 2 : 1);  // outputs of 4 (rope: 2 x 4) columns in a tile
+  static_assert(TM * TN * kLanes <= NW * 64, "one output per thread");
+  const int tile = threadIdx.x / kLanes, l = threadIdx.x % kLanes, ti = tile / TN, tj = tile % TN;
+  const int m = m0 + ti * 16 + (l & 15);
+  const int n = (EPI == kRope ? pair_column(n0 + tj * 16, p.head_dim) : n0 + tj * kCols) + (l >> 4) * 4;
+  const int ldc = EPI == kSilu ? p.n >> 1 : p.n;
+  const bool writes = tile < TM * TN && m < p.m;
+  const int64_t at_out = (static_cast<int64_t>(m) * ldc + n) * 2;
+  E add0[4], add1[4], c0[4], c1[4], s0[4], s1[4];
+  bool rotate = false;
+  if (writes) {
+    if (EPI == kResidual) __builtin_memcpy(add0, p.residual + at_out, 8);
+    if ((EPI == kPlain || EPI == kRope) && p.bias) __builtin_memcpy(add0, p.bias + n * 2, 8);
+    if (EPI == kRope) {
+      if (p.bias) __builtin_memcpy(add1, p.bias + (n + half) * 2, 8);
+      const int head = n / p.head_dim, d = n - head * p.head_dim;
+      rotate = head < p.rot_heads;
+      if (rotate) {
+        const char* cs = p.cos + m * p.cs_st + d * 2;
+        const char* sn = p.sin + m * p.cs_st + d * 2;
+        __builtin_memcpy(c0, cs, 8);
+        __builtin_memcpy(c1, cs + half * 2, 8);
+        __builtin_memcpy(s0, sn, 8);
+        __builtin_memcpy(s1, sn + half * 2, 8);
+      }
+    }
   }
   const char* np = NORM ? p.norm + quad * 16 : nullptr;
 
@@ -215,41 +260,52 @@ __global__ __launch_bounds__(NW * 64) void small_linear_kernel(LinearArgs p) {
     for (int j = 0; j < TN; ++j) part[wave][i * TN + j][lane] = acc[i][j];
   __syncthreads();
 
-  const int ldc = EPI == kSilu ? p.n >> 1 : p.n;
-  auto total = [&](int t, int l) {
-    f32x4 v = part[0][t][l];
+  if (!writes) return;
+  auto total = [&](int at) {
+    f32x4 v = part[0][tile][at];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) v += part[w][t][l];
+    for (int w = 1; w < NW; ++w) v += part[w][tile][at];
     return v;
   };
-  for (int o = threadIdx.x; o < TM * TN * 4 * kCols; o += NW * 64) {
-    const int t = o / (4 * kCols), l = o % (4 * kCols), i = t / TN, j = t % TN;
-    const int m = m0 + i * 16 + (l & 15), n = n0 + j * kCols + (l >> 4) * 4;
-    if (m >= p.m) continue;
-    const int64_t at_out = (static_cast<int64_t>(m) * ldc + n) * 2;
-    f32x4 v = total(t, l);
-    E e[4];
-    auto stored = [](float f) { return static_cast<float>(static_cast<E>(f)); };
-    if (EPI == kSilu) {
-      const f32x4 up = total(t, l + 32);
+  auto stored = [](float f) { return static_cast<float>(static_cast<E>(f)); };
+  f32x4 v = total(l);
+  E e[4];
+  if constexpr (EPI == kSilu) {
+    const f32x4 up = total(l + 32);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float g = stored(v[c]);
+      v[c] = stored(g / (1.f + expf(-g))) * stored(up[c]);
+    }
+  } else if constexpr (EPI == kResidual) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = static_cast<float>(add0[c]) + stored(v[c]);
+  } else if (p.bias) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] += static_cast<float>(add0[c]);
+  }
+  if constexpr (EPI == kRope) {
+    f32x4 x1 = total(l + 32);
+    if (p.bias) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x1[c] += static_cast<float>(add1[c]);
+    }
+    if (rotate) {
+      // The rounding of every product and sum, as rope_append.hip (bit-identical to it).
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const float g = stored(v[c]);
-        v[c] = stored(g / (1.f + expf(-g))) * stored(up[c]);
+        const float a = stored(v[c]), b = stored(x1[c]);
+        v[c] = stored(a * static_cast<float>(c0[c])) + stored(-b * static_cast<float>(s0[c]));
+        x1[c] = stored(b * static_cast<float>(c1[c])) + stored(a * static_cast<float>(s1[c]));
       }
-    } else if (EPI == kResidual) {
-      __builtin_memcpy(e, p.residual + at_out, 8);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) v[c] = static_cast<float>(e[c]) + stored(v[c]);
-    } else if (p.bias) {
-      __builtin_memcpy(e, p.bias + n * 2, 8);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) v[c] += static_cast<float>(e[c]);
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) e[c] = static_cast<E>(v[c]);
-    __builtin_memcpy(p.out + at_out, e, 8);
+    for (int c = 0; c < 4; ++c) e[c] = static_cast<E>(x1[c]);
+    __builtin_memcpy(p.out + at_out + half * 2, e, 8);
   }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) e[c] = static_cast<E>(v[c]);
+  __builtin_memcpy(p.out + at_out, e, 8);
 }
 
 template <int DT, int TM, int TN, int NW, int U, bool NORM, int EPI>
@@ -276,11 +332,20 @@ int check(const void* out, const void* a, const void* w, int32_t m, int32_t n, i
 
 // The tile by rows: enough workgroups to cover the CUs at N = 896 .. 9728 while each reads as few
 // rows of A as that allows (a wavefront's A loads cost as much as its W loads at TM = TN = 1).
+template <int DT, bool NORM, int EPI> int plain_linear(const LinearArgs& p, hipStream_t s) {
+  if constexpr (NORM) {
+    if (p.m > 128 && p.n % 64 == 0) return launch<DT, 2, 4, 8, 2, NORM, EPI>(p, s);
+    if (p.m > 64 && p.n % 32 == 0) return launch<DT, 2, 2, 8, 4, NORM, EPI>(p, s);
+  } else {
+    if (p.m > 192 && p.n % 64 == 0) return launch<DT, 2, 4, 8, 2, NORM, EPI>(p, s);
+    if (p.m > 96 && p.n % 32 == 0) return launch<DT, 2, 2, 8, 2, NORM, EPI>(p, s);
+  }
+  if (p.m > 32 && p.n % 32 == 0) return launch<DT, 1, 2, 4, 7, NORM, EPI>(p, s);
+  return p.k <= 1024 ? launch<DT, 1, 1, 4, 8, NORM, EPI>(p, s) : launch<DT, 1, 1, 8, 4, NORM, EPI>(p, s);
+}
 template <int DT> int norm_linear(const LinearArgs& p, hipStream_t s) {
-  if (p.m > 128 && p.n % 64 == 0) return launch<DT, 2, 4, 8, 2, true, kPlain>(p, s);
-  if (p.m > 64 && p.n % 32 == 0) return launch<DT, 2, 2, 8, 4, true, kPlain>(p, s);
-  if (p.m > 32 && p.n % 32 == 0) return launch<DT, 1, 2, 4, 7, true, kPlain>(p, s);
-  return p.k <= 1024 ? launch<DT, 1, 1, 4, 8, true, kPlain>(p, s) : launch<DT, 1, 1, 8, 4, true, kPlain>(p, s);
+  if (p.cos) return p.norm ? plain_linear<DT, true, kRope>(p, s) : plain_linear<DT, false, kRope>(p, s);
+  return plain_linear<DT, true, kPlain>(p, s);
 }
 template <int DT> int norm_gate_up(const LinearArgs& p, hipStream_t s) {
   if (p.m > 32 && p.n % 64 == 0) return launch<DT, 4, 4, 8, 1, true, kSilu>(p, s);
@@ -324,6 +389,29 @@ extern "C" int mip_norm_linear(void* out, const void* x, const void* norm, float
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == MIP_F16) return gate_up ? norm_gate_up<MIP_F16>(p, s) : norm_linear<MIP_F16>(p, s);
   return gate_up ? norm_gate_up<MIP_BF16>(p, s) : norm_linear<MIP_BF16>(p, s);
+}
+
+extern "C" int mip_qkv_linear(void* out, const void* x, const void* norm, float eps, const void* weight, const void* bias,
+                              const void* cos, const void* sin, int64_t cs_stride_tok, int32_t m, int32_t n, int32_t k,
+                              int32_t head_dim, int32_t rot_heads, int32_t dtype, void* stream) {
+  const int st = check(out, x, weight, m, n, k, dtype);
+  if (st != MIP_OK || m == 0) return st;
+  if (!cos || !sin || head_dim <= 0 || rot_heads < 0 || n % head_dim || rot_heads > n / head_dim) return MIP_EINVAL;
+  if (head_dim % 16 || !aligned16(norm) || !aligned16(bias)) return MIP_EUNSUPPORTED;
+  if ((reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin) | static_cast<uint64_t>(cs_stride_tok * 2)) & 7)
+    return MIP_EUNSUPPORTED;  // read 4 elements at a time
+  LinearArgs p = args(out, x, weight, m, n, k);
+  p.norm = static_cast<const char*>(norm);
+  p.bias = static_cast<const char*>(bias);
+  p.cos = static_cast<const char*>(cos);
+  p.sin = static_cast<const char*>(sin);
+  p.cs_st = cs_stride_tok * 2;
+  p.head_dim = head_dim;
+  p.rot_heads = rot_heads;
+  p.eps = eps;
+  p.inv_k = 1.f / static_cast<float>(k);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == MIP_F16 ? norm_linear<MIP_F16>(p, s) : norm_linear<MIP_BF16>(p, s);
 }
 
 extern "C" int mip_linear_residual(void* out, const void* a, const void* weight, const void* residual, int32_t m, int32_t n,

@@ -41,6 +41,7 @@ EXPORTED = (
     "mip_add_rms_norm",
     "mip_silu_mul",
     "mip_norm_linear",
+    "mip_qkv_linear",
     "mip_linear_residual",
 )
 
@@ -134,6 +135,7 @@ _SIGNATURES = {
     "mip_add_rms_norm": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _f32, _i32, _vp]),
     "mip_silu_mul": (_c.c_int, [_vp, _vp, _i32, _i32, _i32, _vp]),
     "mip_norm_linear": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
+    "mip_qkv_linear": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
     "mip_linear_residual": (_c.c_int, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp]),
     "mip_hbm_read_probe": (_c.c_int, [_vp, _i64, _vp, _i64, _i32, _vp, _i32, _i32, _vp]),
 }

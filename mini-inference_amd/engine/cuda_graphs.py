@@ -62,6 +62,7 @@ class _GraphDecodeContext:
         self.scale = 1.0 / (owner.cache.head_dim ** 0.5)
         self.num_heads = owner.model.cfg.num_heads
         self.fuse_rope = owner.fuse_rope
+        self.takes_rotated = True
         # Buffer of the step's work plan; prepare() fills it inside the graph. (The launch is
         # issued there, not prepared here, so that it binds the capturing stream.)
         self.plan = paged_ops.prepare_decode_plan(self.context_lens, self.tables, self.num_heads,

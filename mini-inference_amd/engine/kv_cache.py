@@ -378,7 +378,6 @@ class PagedDecodeContext:
     """
 
     fuse_rope = True
-
     def __init__(self, cache: PagedKVCache, slots: Sequence[int]) -> None:
         self.cache = cache
         self.slots = list(slots)
@@ -423,6 +422,14 @@ class PagedDecodeContext:
         self._mask: torch.Tensor | None = None
         self._plan: tuple[tuple, torch.Tensor | None] | None = None  # (shape key, work plan)
         self._calls: paged_ops.DecodeStepCalls | None = None
+
+    @property
+    def takes_rotated(self) -> bool:
+        """``attend`` appends within the decode call, so rotated q and k save the kernel that ``attend_rope``
+        runs ahead of it. (Not where somebody else's ``attend`` or ``attend_rope`` is to be called.)"""
+        cls = type(self)
+        return (cls.attend is PagedDecodeContext.attend and cls.attend_rope is PagedDecodeContext.attend_rope
+                and "attend" not in self.__dict__ and "attend_rope" not in self.__dict__)
 
     @property
     def tables(self) -> torch.Tensor:

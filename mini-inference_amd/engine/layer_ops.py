@@ -122,6 +122,11 @@ def norm_linear_pays(rows: int, weight: torch.Tensor) -> bool:
     return _linear_fits(rows, weight) and weight.numel() <= limit
 
 
+def qkv_linear_pays(rows: int, weight: torch.Tensor, normed: bool) -> bool:
+    """As :func:`norm_linear_pays`, without the library's separate rotary kernel; ``normed``: x is normed already."""
+    return norm_linear_pays(rows, weight) or (normed and _linear_fits(rows, weight) and weight.numel() <= 3 << 19)
+
+
 def norm_gate_up_pays(rows: int, weight: torch.Tensor) -> bool:
     limit = 48 << 20 if rows <= 16 else 12 << 20 if rows <= 64 else 0
     return _linear_fits(rows, weight) and weight.numel() <= limit
@@ -147,6 +152,29 @@ def norm_linear(x: torch.Tensor, norm: torch.Tensor, eps: float, weight: torch.T
                                         _DTYPE_CODES[x.dtype], _stream_ptr(x.device))
     if st:
         _native.check(st, "mip_norm_linear")
+    return out
+
+
+def rope_usable(cos: torch.Tensor, sin: torch.Tensor, x: torch.Tensor, head_dim: int) -> bool:
+    """Whether :func:`qkv_linear` can take these rotary tables for rows ``x [B, T, hidden]``."""
+    return (cos.shape == sin.shape == (x.shape[0], 1, x.shape[1], head_dim) and head_dim % 16 == 0
+            and usable(x, cos, sin))
+
+
+def qkv_linear(x: torch.Tensor, norm: torch.Tensor | None, eps: float, weight: torch.Tensor, bias: torch.Tensor | None,
+               cos: torch.Tensor, sin: torch.Tensor, rot_heads: int) -> torch.Tensor:
+    """:func:`norm_linear` (of x itself where ``norm`` is None) with the rotary embedding applied to the first
+    ``rot_heads`` heads of its output; cos, sin ``[B, 1, T, head_dim]``. The rotation is
+    :func:`engine.paged_ops.rope_kv_append`'s, bit for bit."""
+    n, k = weight.shape
+    d = cos.shape[-1]
+    out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    st = _native.load().mip_qkv_linear(out.data_ptr(), x.data_ptr(), None if norm is None else norm.data_ptr(), eps,
+                                       weight.data_ptr(), None if bias is None else bias.data_ptr(), cos.data_ptr(),
+                                       sin.data_ptr(), d, x.numel() // k, n, k, d, rot_heads, _DTYPE_CODES[x.dtype],
+                                       _stream_ptr(x.device))
+    if st:
+        _native.check(st, "mip_qkv_linear")
     return out
 
 

@@ -69,7 +69,9 @@ class AttentionContext(Protocol):
 
     A context whose ``fuse_rope`` attribute is true instead receives q and k before the
     rotary embedding, with the step's cos/sin tables, through
-    ``attend_rope(layer_idx, q, k, v, cos, sin)``, and applies the rotation itself.
+    ``attend_rope(layer_idx, q, k, v, cos, sin)``, and applies the rotation itself. One whose
+    ``takes_rotated`` attribute is true as well may be given rotated q and k through ``attend``
+    instead, where the layer has a cheaper place for the rotation (the end of its projection).
     """
 
     def attend(self, layer_idx: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor: ...
@@ -131,15 +133,19 @@ class Attention(nn.Module):
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, ctx: AttentionContext) -> torch.Tensor:
         return self.o_proj(self.attend(self.qkv_proj(x), cos, sin, ctx))
 
-    def attend(self, qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, ctx: AttentionContext) -> torch.Tensor:
-        """The part between the projections: ``[B, T, q + 2 kv]`` in, ``[B, T, q]`` out."""
+    def attend(self, qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, ctx: AttentionContext,
+               rotated: bool = False) -> torch.Tensor:
+        """The part between the projections: ``[B, T, q + 2 kv]`` in, ``[B, T, q]`` out. ``rotated``: the rotary
+        embedding has been applied."""
         c = self.cfg
         bsz, t, _ = qkv.shape
         q, k, v = qkv.split([c.q_size, c.kv_size, c.kv_size], dim=-1)
         q = q.view(bsz, t, c.num_heads, c.head_dim).transpose(1, 2)
         k = k.view(bsz, t, c.num_kv_heads, c.head_dim).transpose(1, 2)
         v = v.view(bsz, t, c.num_kv_heads, c.head_dim).transpose(1, 2)
-        if getattr(ctx, "fuse_rope", False):
+        if rotated:
+            out = ctx.attend(self.layer_idx, q, k, v)
+        elif getattr(ctx, "fuse_rope", False):
             # The context rotates q and k itself (in place), fused with its KV append.
             out = ctx.attend_rope(self.layer_idx, q, k, v, cos, sin)
         else:
@@ -203,15 +209,24 @@ class DecoderLayer(nn.Module):
         """
         a, m, n1, n2 = self.attn, self.mlp, self.input_norm, self.post_attn_norm
         rows = x.shape[0] * x.shape[1]
-        w = a.qkv_proj.weight
+        w, c = a.qkv_proj.weight, a.cfg
+        normed = None
         if delta is not None:
             x, normed = layer_ops.add_rms_norm(x, delta, n1.weight, n1.eps)
+        # A context that takes rotated q and k in its fused append gets them from the projection itself.
+        rotated = (getattr(ctx, "fuse_rope", False) and getattr(ctx, "takes_rotated", False)
+                   and layer_ops.qkv_linear_pays(rows, w, normed is not None)
+                   and layer_ops.rope_usable(cos, sin, x, c.head_dim))
+        if rotated:
+            src, norm = (x, n1.weight) if normed is None else (normed, None)
+            qkv = layer_ops.qkv_linear(src, norm, n1.eps, w, a.qkv_proj.bias, cos, sin, c.num_heads + c.num_kv_heads)
+        elif normed is not None:
             qkv = F.linear(normed, w, a.qkv_proj.bias)
         elif layer_ops.norm_linear_pays(rows, w):
             qkv = layer_ops.norm_linear(x, n1.weight, n1.eps, w, a.qkv_proj.bias)
         else:
             qkv = F.linear(layer_ops.rms_norm(x, n1.weight, n1.eps), w, a.qkv_proj.bias)
-        out, w = a.attend(qkv, cos, sin, ctx), a.o_proj.weight
+        out, w = a.attend(qkv, cos, sin, ctx, rotated), a.o_proj.weight
         if out.shape[:2] != x.shape[:2] or not layer_ops.usable(x, out):  # a context with outputs of its own kind
             x = x + F.linear(out, w)
             return x + m(n2(x)), None

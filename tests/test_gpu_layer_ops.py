@@ -149,7 +149,8 @@ def test_routes_that_stay_on_torch(gpu):
 # leave a single 16-column tile, an odd number of tiles, fewer k-steps than wavefronts, k-steps that do
 # not divide among them, and the 0.5B model's own shapes.
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("n,k", [(16, 32), (48, 96), (80, 1056), (1152, 896), (896, 4864), (2080, 160)])
+@pytest.mark.parametrize("n,k", [(16, 32), (48, 96), (80, 1056), (64, 1152), (32, 2112), (1152, 896), (896, 4864),
+                                 (2080, 160)])
 def test_small_linears(gpu, dtype, n, k):
     from engine import layer_ops
 
@@ -235,3 +236,102 @@ def test_fused_layer_matches_its_modules(gpu, dtype):
             # Both round each intermediate once or twice: a few roundings of relative size U each.
             err = (got.double() - want.double()).norm() / want.double().norm()
             assert err <= 8 * U[dtype], (hidden, b, t, float(err))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,hq,hkv,k", [(64, 14, 2, 896), (128, 4, 2, 192), (16, 3, 1, 64), (32, 1, 3, 1056),
+                                          (64, 2, 1, 2112)])
+def test_qkv_linear_rotates_as_the_rope_kernel(gpu, dtype, d, hq, hkv, k):
+    """The projection with the rotation inside: bit-equal to the projection, then rope_kv_append's rotation."""
+    from engine import layer_ops, paged_ops
+    from engine.model import rope_cos_sin
+
+    for m in (1, 8, 17, 33, 64, 65, 130, 256):
+        announce(f"qkv_linear {dtype} d={d} hq={hq} hkv={hkv} k={k} m={m}")
+        gen = torch.Generator(device=gpu).manual_seed(m + d)
+        n = (hq + 2 * hkv) * d
+        x = torch.randn(m, 1, k, generator=gen, device=gpu).to(dtype)
+        w = (torch.randn(n, k, generator=gen, device=gpu) / k ** 0.5).to(dtype)
+        norm = (torch.rand(k, generator=gen, device=gpu) + 0.5).to(dtype)
+        bias = torch.randn(n, generator=gen, device=gpu).to(dtype)
+        pos = torch.randint(0, 4096, (m, 1), generator=gen, device=gpu)
+        cos, sin = rope_cos_sin(pos, d, 1e6, dtype)
+        assert layer_ops.rope_usable(cos, sin, x, d)
+        pool = torch.zeros(1, hkv, 1, d, dtype=dtype, device=gpu)
+        skip = torch.full((m,), -1, dtype=torch.int64, device=gpu)
+
+        def rotate(y):
+            y = y.clone().view(m, hq + 2 * hkv, d)
+            paged_ops.rope_kv_append(y[:, :hq], y[:, hq:hq + hkv], y[:, hq + hkv:], cos[:, 0, 0], sin[:, 0, 0], pool,
+                                     pool.clone(), skip)
+            return y.view(m, 1, n)
+
+        got = layer_ops.qkv_linear(x, norm, 1e-6, w, bias, cos, sin, hq + hkv)
+        if m <= 64:  # the same tiles, so the same sums
+            assert torch.equal(got, rotate(layer_ops.norm_linear(x, norm, 1e-6, w, bias)))
+        # Of x as it is, and with no head rotated: the projection itself, rotated afterwards.
+        plain = layer_ops.qkv_linear(x, None, 0.0, w, bias, cos, sin, 0)
+        want = (x.double() @ w.double().t() + bias.double()).view(m, 1, n)
+        mag = x.double().abs() @ w.double().abs().t()
+        assert ((plain.double() - want).abs() <= 1.01 * U[dtype] * want.abs() + (k / 64 + 8) * 2 ** -24 * mag + TINY).all()
+        assert torch.equal(layer_ops.qkv_linear(x, None, 0.0, w, bias, cos, sin, hq + hkv), rotate(plain))
+        bare = layer_ops.qkv_linear(x, norm, 1e-6, w, None, cos, sin, hq + hkv)
+        assert torch.isfinite(bare.float()).all() and bare.shape == got.shape
+
+
+@torch.inference_mode()
+def test_contexts_that_rotate_for_themselves_still_do(gpu):
+    """A decode context's own attend_rope, wrapped, subclassed or patched, is called where there is one."""
+    from engine.kv_cache import PagedDecodeContext, PagedKVCache
+    from engine.model import DecoderLayer, Qwen2Config, rope_cos_sin
+
+    announce("takes_rotated: wrapped and subclassed contexts")
+    cfg = Qwen2Config(vocab_size=64, hidden_size=256, intermediate_size=512, num_layers=1, num_heads=4, num_kv_heads=2,
+                      head_dim=64)
+    dt = torch.bfloat16
+    layer = DecoderLayer(cfg, 0).to(gpu).to(dt).requires_grad_(False)
+    cache = PagedKVCache(1, 2, 64, 64, 16, max_seqs=8, max_len=256, dtype=dt, device=gpu)
+    slots = []
+    for n in (5, 33, 100):
+        s = cache.allocate(n + 1)
+        cache.lengths[s] = n
+        slots.append(s)
+    cache.k.normal_()
+    cache.v.normal_()
+    k0, v0 = cache.k.clone(), cache.v.clone()
+    x = torch.randn(3, 1, 256, device=gpu).to(dt)
+    calls = []
+
+    class Sub(PagedDecodeContext):
+        def attend_rope(self, *a):
+            calls.append("sub")
+            return super().attend_rope(*a)
+
+    class Wrap:
+        fuse_rope = True
+
+        def __init__(self, inner):
+            self.inner = inner
+
+        def attend_rope(self, *a):
+            calls.append("wrap")
+            return self.inner.attend_rope(*a)
+
+    def run(ctx, inner):
+        cache.k.copy_(k0)
+        cache.v.copy_(v0)
+        cos, sin = rope_cos_sin(inner.positions.unsqueeze(1), 64, cfg.rope_theta, dt)
+        return layer(x, cos, sin, ctx), cache.k.clone(), cache.v.clone()
+
+    inner = PagedDecodeContext(cache, slots)
+    assert inner.takes_rotated
+    want = run(inner, inner)
+    sub = Sub(cache, slots)
+    assert not sub.takes_rotated
+    inner2 = PagedDecodeContext(cache, slots)
+    inner3 = PagedDecodeContext(cache, slots)
+    inner3.fuse_rope = False
+    for ctx, base in ((sub, sub), (Wrap(inner2), inner2), (inner3, inner3)):
+        for a, b in zip(run(ctx, base), want):
+            assert torch.equal(a, b)
+    assert calls == ["sub", "wrap"]

@@ -401,6 +401,28 @@ int mip_linear_residual(void* out, const void* a, const void* weight, const void
                         int32_t n, int32_t k, int32_t dtype, void* stream);
 
 /*
+ * The inputs of a decode step from device-resident tables (engine/kv_cache.py:592-609), two launches:
+ * rows[journal_flat[i]] = journal_block[i] for the n_journal entries (rows taken flat; an index that
+ * occurs twice has to carry one value), then for each sequence b of the batch, with p = positions[b]:
+ *     tables[b * table_stride + i] = rows[row_ids[b] * row_stride + i]      i < n_blocks
+ *     slot_mapping[b] = rows[row_ids[b] * row_stride + p / block_size] * block_size + p % block_size
+ *     context_lens[b] = p + 1
+ * Every index must lie inside rows, and p / block_size below n_blocks.
+ */
+int mip_decode_prepare(int32_t* rows, int64_t row_stride, const int64_t* journal_flat, const int64_t* journal_block,
+                       int32_t n_journal, const int64_t* row_ids, const int64_t* positions, int32_t* tables,
+                       int64_t table_stride, int32_t n_blocks, int64_t* slot_mapping, int32_t* context_lens,
+                       int32_t batch, int32_t block_size, void* stream);
+
+/*
+ * Rotary tables (engine/model.py:205-213): for token t and j < head_dim / 2, with the angle
+ * positions[t] / theta^(2 j / head_dim) evaluated in fp32, cos[t][j] = cos[t][j + head_dim / 2] = its
+ * cosine and sin alike, rounded to dtype; rows of head_dim contiguous elements.
+ */
+int mip_rope_tables(void* cos, void* sin, const int64_t* positions, int32_t n_tokens, int32_t head_dim, float theta,
+                    int32_t dtype, void* stream);
+
+/*
  * The layer calls of one step. Every layer of a step passes the same sequences, strides and sizes
  * and other tensors of the same layout; these entry points take what stays the same as a host
  * struct (read during the call, owned by the caller) and the layer's pointers as arguments. Each is

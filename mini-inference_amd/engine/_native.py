@@ -33,6 +33,8 @@ EXPORTED = (
     "mip_copy_blocks",
     "mip_copy_blocks_host",
     "mip_prefill_index",
+    "mip_decode_prepare",
+    "mip_rope_tables",
     "mip_decode_step_append",
     "mip_decode_step_attend",
     "mip_rope_step_append",
@@ -129,6 +131,8 @@ _SIGNATURES = {
     "mip_rope_step_append": (_c.c_int, [_vp] * 9),
     "mip_prefill_step_append": (_c.c_int, [_vp] * 6),
     "mip_prefill_step_attend": (_c.c_int, [_vp] * 6),
+    "mip_decode_prepare": (_c.c_int, [_vp, _i64, _vp, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _vp, _vp, _i32, _i32, _vp]),
+    "mip_rope_tables": (_c.c_int, [_vp, _vp, _vp, _i32, _i32, _f32, _i32, _vp]),
     "mip_prefill_index": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp]),
     "mip_copy_blocks": (_c.c_int, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp]),
     "mip_copy_blocks_host": (_c.c_int, [_vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp]),

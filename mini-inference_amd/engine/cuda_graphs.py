@@ -73,13 +73,10 @@ class _GraphDecodeContext:
     def prepare(self) -> None:
         """Inside the graph, once per step: table updates, the batch's rows, slot mapping, context lengths."""
         owner = self.owner
-        rows = owner.device_tables.rows
-        rows.view(-1).scatter_(0, owner.journal_flat, owner.journal_block.to(torch.int32))
-        torch.index_select(rows, 0, owner.row_ids[:self.batch], out=owner.tables[:self.batch])
-        bs = self.cache.block_size
-        write_blocks = self.tables.gather(1, torch.div(self.positions, bs, rounding_mode="floor").unsqueeze(1))
-        self.slot_mapping.copy_(write_blocks.squeeze(1).to(torch.int64) * bs + self.positions % bs)
-        self.context_lens.copy_(self.positions + 1)
+        paged_ops.decode_prepare(owner.device_tables.rows, owner.journal_flat, owner.journal_block,
+                                 owner.row_ids[:self.batch], self.positions, owner.tables[:self.batch],
+                                 owner.device_tables.max_blocks, self.slot_mapping, self.context_lens,
+                                 self.cache.block_size)
         if self.plan is not None:
             c = self.cache
             paged_ops.decode_plan(self.context_lens, self.tables, self.num_heads, c.num_kv_heads, c.head_dim,

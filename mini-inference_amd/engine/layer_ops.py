@@ -78,6 +78,23 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
     return s, out
 
 
+def rope_tables(positions: torch.Tensor, head_dim: int, theta: float,
+                dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor] | None:
+    """cos/sin ``[B, 1, T, D]`` for ``positions [B, T]`` in one launch, or None where it does not apply."""
+    if (not positions.is_cuda or type(positions) is not torch.Tensor or positions.dtype != torch.int64
+            or positions.dim() != 2 or not positions.is_contiguous() or dtype not in _DTYPE_CODES or head_dim % 2
+            or type(theta) not in (float, int) or theta <= 0 or not 0 < positions.numel() * head_dim < 1 << 31
+            or positions.device.index != torch.cuda.current_device() or _observed()):
+        return None
+    b, t = positions.shape
+    cos, sin = (torch.empty((b, 1, t, head_dim), dtype=dtype, device=positions.device) for _ in range(2))
+    st = _native.load().mip_rope_tables(cos.data_ptr(), sin.data_ptr(), positions.data_ptr(), b * t, head_dim, theta,
+                                        _DTYPE_CODES[dtype], _stream_ptr(positions.device))
+    if st:
+        _native.check(st, "mip_rope_tables")
+    return cos, sin
+
+
 def silu_mul_usable(gate_up: torch.Tensor) -> bool:
     if gate_up.dim() < 1 or gate_up.shape[-1] % 2 or gate_up.numel() == 0:
         return False

@@ -107,6 +107,9 @@ class RMSNorm(nn.Module):
 
 def rope_cos_sin(positions: torch.Tensor, head_dim: int, theta: float, dtype: torch.dtype):
     """cos/sin ``[B, 1, T, D]`` for per-token ``positions [B, T]`` (half-rotation layout)."""
+    tables = layer_ops.rope_tables(positions, head_dim, theta, dtype)
+    if tables is not None:
+        return tables
     half = head_dim // 2
     inv_freq = 1.0 / (theta ** (torch.arange(half, device=positions.device, dtype=torch.float32) * 2.0 / head_dim))
     ang = positions.to(torch.float32).unsqueeze(-1) * inv_freq  # [B, T, D/2]

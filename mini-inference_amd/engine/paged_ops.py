@@ -541,6 +541,32 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
     return out
 
 
+def decode_prepare(rows: torch.Tensor, journal_flat: torch.Tensor, journal_block: torch.Tensor, row_ids: torch.Tensor,
+                   positions: torch.Tensor, tables: torch.Tensor, n_blocks: int, slot_mapping: torch.Tensor,
+                   context_lens: torch.Tensor, block_size: int) -> None:
+    """A decode step's inputs from the device mirror of the block tables (``mip_decode_prepare``): apply the journal
+    to ``rows``, gather the batch's first ``n_blocks`` entries into ``tables``, and write each new token's slot and
+    each sequence's length."""
+    _require_device(rows, journal_flat, journal_block, row_ids, positions, tables, slot_mapping, context_lens)
+    for t in (journal_flat, journal_block, row_ids, positions, slot_mapping):
+        if t.dtype != torch.int64 or t.dim() != 1 or not t.is_contiguous():
+            raise ValueError("journal, row ids, positions and slots must be contiguous int64 vectors")
+    if rows.dtype != torch.int32 or not rows.is_contiguous() or tables.dtype != torch.int32 or tables.stride(1) != 1:
+        raise ValueError("rows and tables must be int32 with contiguous rows")
+    b = row_ids.shape[0]
+    if (journal_flat.shape != journal_block.shape or positions.shape[0] != b or slot_mapping.shape[0] != b
+            or context_lens.shape != (b,) or context_lens.dtype != torch.int32 or not context_lens.is_contiguous()
+            or tables.shape[0] < b or min(tables.shape[1], rows.shape[1]) < n_blocks):
+        raise ValueError("decode_prepare: the batch's tensors do not match")
+    st = _native.load().mip_decode_prepare(rows.data_ptr(), rows.stride(0), journal_flat.data_ptr(),
+                                           journal_block.data_ptr(), journal_flat.shape[0], row_ids.data_ptr(),
+                                           positions.data_ptr(), tables.data_ptr(), tables.stride(0), n_blocks,
+                                           slot_mapping.data_ptr(), context_lens.data_ptr(), b, block_size,
+                                           _stream_ptr(rows.device))
+    if st:
+        _native.check(st, "mip_decode_prepare")
+
+
 def prefill_index(cu_q: torch.Tensor, ctx_start: torch.Tensor, block_tables: torch.Tensor, n_tokens: int,
                   max_q_len: int, block_size: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """``positions`` and ``slot_mapping`` (int64 ``[n_tokens]``) of a packed prefill step's new tokens, and

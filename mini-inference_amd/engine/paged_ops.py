@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+from itertools import chain
 
 import numpy as np
 import torch
@@ -661,7 +662,10 @@ def paged_decode_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cac
 def _copy_shape(k_pool: torch.Tensor, v_pool: torch.Tensor) -> tuple[int, int, int]:
     if k_pool.shape != v_pool.shape or k_pool.dim() != 5 or not (k_pool.is_contiguous() and v_pool.is_contiguous()):
         raise ValueError("k_pool/v_pool must be contiguous [L, num_blocks, Hkv, block_size, D] tensors of one shape")
-    return k_pool.shape[0], k_pool.shape[1], k_pool[0, 0].numel() * k_pool.element_size()
+    layers, blocks, heads, block_size, dim = k_pool.shape
+    if layers == 0 or blocks == 0:
+        raise IndexError("the pool holds no blocks")
+    return layers, blocks, heads * block_size * dim * k_pool.element_size()
 
 
 def _host_pairs(pairs) -> np.ndarray:
@@ -669,6 +673,9 @@ def _host_pairs(pairs) -> np.ndarray:
     sequence of (src, dst)), so a prepared call keeps the pairs it was prepared with."""
     if isinstance(pairs, torch.Tensor):
         pairs = pairs.numpy()
+    elif type(pairs) is list and set(map(type, pairs)) == {tuple} and set(map(len, pairs)) == {2}:
+        # What prepare_writes builds: read flat, a third of the time of the nested conversion.
+        return np.fromiter(chain.from_iterable(pairs), np.int64, 2 * len(pairs)).reshape(-1, 2)
     return np.array(pairs, dtype=np.int64, copy=True, order="C").reshape(-1, 2)
 
 

@@ -20,39 +20,48 @@ _MAX_ROW_BYTES = 32768
 
 def _observed() -> bool:
     """Whether something other than the plain eager dispatch would see a torch op called now."""
-    return (torch._C._len_torch_function_stack() > 0 or torch._C._len_torch_dispatch_stack() > 0
+    return (torch.compiler.is_compiling()  # first: a compiler that traces this function stops reading here
+            or torch._C._len_torch_function_stack() > 0 or torch._C._len_torch_dispatch_stack() > 0
             or torch._C._functorch.peek_interpreter_stack() is not None or _FWD_AD._current_level >= 0
-            or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
-            or torch.is_autocast_enabled("cuda"))
+            or torch._C._get_tracing_state() is not None or torch.is_autocast_enabled("cuda"))
 
 
-def usable(*tensors: torch.Tensor) -> bool:
-    """Whether the fused kernels may take these operands (16-byte aligned, dense, one dtype and device)."""
-    x = tensors[0]
-    if not x.is_cuda or x.dtype not in _DTYPE_CODES or _observed():
-        return False
+def _open(x: torch.Tensor) -> bool:
+    """Whether this device tensor's op may be taken over at all (asked before anything about its sizes)."""
+    return x.is_cuda and x.dtype in _DTYPE_CODES and not _observed()
+
+
+def _operands(x: torch.Tensor, *others: torch.Tensor) -> bool:
+    """Whether the kernels can read these: dense, 16-byte aligned, one dtype, on the current device, no gradient."""
     grad = torch.is_grad_enabled()
-    for t in tensors:
+    for t in (x, *others):
         if (type(t) not in _PLAIN or t.dtype != x.dtype or t.device != x.device or not t.is_contiguous()
                 or t.data_ptr() % 16 or (grad and t.requires_grad) or t.is_neg()):
             return False
     return x.device.index == torch.cuda.current_device()
 
 
-def _row_ok(t: torch.Tensor, limit: int | None = None) -> bool:
+def usable(x: torch.Tensor, *others: torch.Tensor) -> bool:
+    """Whether the fused kernels may take these operands."""
+    return _open(x) and _operands(x, *others)
+
+
+def _row_ok(t: torch.Tensor, limit: int) -> bool:
     if t.dim() < 1 or t.numel() == 0:
         return False
     nbytes = t.shape[-1] * t.element_size()
-    return nbytes % 16 == 0 and (limit is None or nbytes <= limit) and t.numel() // t.shape[-1] < 1 << 31
+    return nbytes % 16 == 0 and nbytes <= limit and t.numel() // t.shape[-1] < 1 << 31
 
 
 def norm_usable(weight: torch.Tensor, x: torch.Tensor, delta: torch.Tensor | None = None) -> bool:
     """Whether :func:`add_rms_norm` / :func:`rms_norm` take these (``delta`` of x's own shape)."""
+    if not _open(x):
+        return False
     if weight.dim() != 1 or x.dim() < 1 or weight.shape[0] != x.shape[-1] or not _row_ok(x, _MAX_ROW_BYTES):
         return False
     if delta is None:
-        return usable(x, weight)
-    return delta.shape == x.shape and usable(x, delta, weight)
+        return _operands(x, weight)
+    return delta.shape == x.shape and _operands(x, delta, weight)
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -81,10 +90,10 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
 def rope_tables(positions: torch.Tensor, head_dim: int, theta: float,
                 dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor] | None:
     """cos/sin ``[B, 1, T, D]`` for ``positions [B, T]`` in one launch, or None where it does not apply."""
-    if (not positions.is_cuda or type(positions) is not torch.Tensor or positions.dtype != torch.int64
+    if (not positions.is_cuda or _observed() or type(positions) is not torch.Tensor or positions.dtype != torch.int64
             or positions.dim() != 2 or not positions.is_contiguous() or dtype not in _DTYPE_CODES or head_dim % 2
             or type(theta) not in (float, int) or theta <= 0 or not 0 < positions.numel() * head_dim < 1 << 31
-            or positions.device.index != torch.cuda.current_device() or _observed()):
+            or positions.device.index != torch.cuda.current_device()):
         return None
     b, t = positions.shape
     cos, sin = (torch.empty((b, 1, t, head_dim), dtype=dtype, device=positions.device) for _ in range(2))
@@ -96,10 +105,10 @@ def rope_tables(positions: torch.Tensor, head_dim: int, theta: float,
 
 
 def silu_mul_usable(gate_up: torch.Tensor) -> bool:
-    if gate_up.dim() < 1 or gate_up.shape[-1] % 2 or gate_up.numel() == 0:
+    if not _open(gate_up) or gate_up.dim() < 1 or gate_up.shape[-1] % 2 or gate_up.numel() == 0:
         return False
     half = gate_up.shape[-1] // 2 * gate_up.element_size()
-    return half % 16 == 0 and gate_up.numel() * gate_up.element_size() // 32 < 1 << 31 and usable(gate_up)
+    return half % 16 == 0 and gate_up.numel() * gate_up.element_size() // 32 < 1 << 31 and _operands(gate_up)
 
 
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:

@@ -82,6 +82,8 @@ def _plain(module: nn.Module, cls: type) -> bool:
 
     A fused step that passes a submodule's call by is only taken where nobody watches that call.
     """
+    if torch.compiler.is_compiling():
+        return False
     g = nn.modules.module
     return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
             and not module._forward_pre_hooks and not module._backward_hooks and not module._backward_pre_hooks
@@ -98,8 +100,9 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if layer_ops.norm_usable(self.weight, x):
-            return layer_ops.rms_norm(x, self.weight, self.eps)
+        if not torch.jit.is_scripting():
+            if layer_ops.norm_usable(self.weight, x):
+                return layer_ops.rms_norm(x, self.weight, self.eps)
         xf = x.float()
         inv = torch.rsqrt(xf.square().mean(dim=-1, keepdim=True) + self.eps)
         return self.weight * (xf * inv).to(x.dtype)
@@ -107,9 +110,10 @@ class RMSNorm(nn.Module):
 
 def rope_cos_sin(positions: torch.Tensor, head_dim: int, theta: float, dtype: torch.dtype):
     """cos/sin ``[B, 1, T, D]`` for per-token ``positions [B, T]`` (half-rotation layout)."""
-    tables = layer_ops.rope_tables(positions, head_dim, theta, dtype)
-    if tables is not None:
-        return tables
+    if not torch.jit.is_scripting():
+        tables = layer_ops.rope_tables(positions, head_dim, theta, dtype)
+        if tables is not None:
+            return tables
     half = head_dim // 2
     inv_freq = 1.0 / (theta ** (torch.arange(half, device=positions.device, dtype=torch.float32) * 2.0 / head_dim))
     ang = positions.to(torch.float32).unsqueeze(-1) * inv_freq  # [B, T, D/2]
@@ -166,10 +170,10 @@ class MLP(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.down_proj(self.gated(self.gate_up_proj(x)))
 
-    @staticmethod
-    def gated(gate_up: torch.Tensor) -> torch.Tensor:
-        if layer_ops.silu_mul_usable(gate_up):
-            return layer_ops.silu_mul(gate_up)
+    def gated(self, gate_up: torch.Tensor) -> torch.Tensor:
+        if not torch.jit.is_scripting():
+            if layer_ops.silu_mul_usable(gate_up):
+                return layer_ops.silu_mul(gate_up)
         gate, up = gate_up.chunk(2, dim=-1)
         return F.silu(gate) * up
 

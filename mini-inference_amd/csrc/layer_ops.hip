@@ -15,6 +15,11 @@
 // read twice: one wavefront per row up to 256 16-byte chunks (no barrier, no LDS; 4 rows per
 // workgroup), four wavefronts per row above that, since one lane would otherwise hold more
 // than 4 chunks of x and of delta and the row's loads would queue on a single wavefront.
+//
+// Measured at the 0.5B widths, bf16: 3,924 rows, add + norm 9.2 us (28 MB), norm alone 5.6, gating
+// 22.4 us (115 MB, 5.1 TB/s), where torch's elementwise kernels of one layer took about 150 us; at 8
+// rows 3.8 to 4.0 us each, the launch (torch: 7 launches of 2 to 5 us per norm). One row per
+// 64-thread workgroup at 256 rows: 5.0 us, no different from 4 rows per workgroup.
 #include "mip_common.h"
 
 namespace mip {

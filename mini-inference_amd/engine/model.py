@@ -200,11 +200,13 @@ class DecoderLayer(nn.Module):
         linears = (a.qkv_proj, a.o_proj, m.gate_up_proj, m.down_proj)
         if not all(_plain(p, nn.Linear) for p in linears) or any(p.bias is not None for p in linears[1:]):
             return False
-        w = [p.weight for p in linears] + ([a.qkv_proj.bias] if a.qkv_proj.bias is not None else [])
-        h = x.shape[-1]
-        return (x.dim() == 3 and w[0].shape[1] == h and w[1].shape[0] == h and w[2].shape[1] == h
-                and w[3].shape == (h, w[2].shape[0] // 2) and n2.weight.shape == n1.weight.shape
-                and layer_ops.norm_usable(n1.weight, x) and layer_ops.usable(x, n2.weight, *w))
+        w, bias, c = [p.weight for p in linears], a.qkv_proj.bias, a.cfg
+        h, qkv, inter = x.shape[-1], c.q_size + 2 * c.kv_size, w[2].shape[0] // 2
+        # Every width: the kernels take a shape that torch would refuse for a longer list of rows.
+        return (x.dim() == 3 and w[0].shape == (qkv, h) and w[1].shape == (h, c.q_size) and w[2].shape == (2 * inter, h)
+                and w[3].shape == (h, inter) and (bias is None or bias.shape == (qkv,))
+                and n2.weight.shape == n1.weight.shape and layer_ops.norm_usable(n1.weight, x)
+                and layer_ops.usable(x, n2.weight, *w, *(() if bias is None else (bias,))))
 
     def _fused(self, x, delta, cos, sin, ctx, whole=False):
         """``forward`` of ``x + delta`` (None: of x), as ``(y, delta)`` whose sum it is (None: y is).

@@ -3,7 +3,8 @@
 ``usable`` is the rule: plain contiguous tensors of one supported dtype on the current ROCm
 device, with nothing recording, transforming or tracing the call. Everything else (CPU tensors,
 autograd, torch.func, autocast, tensor subclasses, odd layouts) keeps the torch ops, which
-compute the same values.
+compute the same values. Each function checks its operands on the host and raises for those
+that its kernel cannot read.
 """
 
 from __future__ import annotations
@@ -11,7 +12,7 @@ from __future__ import annotations
 import torch
 
 from . import _native
-from .paged_ops import _DTYPE_CODES, _stream_ptr
+from .paged_ops import _DTYPE_CODES, _require_device, _stream_ptr, dtype_code
 
 _FWD_AD = torch.autograd.forward_ad
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
@@ -64,8 +65,31 @@ def norm_usable(weight: torch.Tensor, x: torch.Tensor, delta: torch.Tensor | Non
     return delta.shape == x.shape and _operands(x, delta, weight)
 
 
+def _check(what: str, fits: bool, x: torch.Tensor, *others: torch.Tensor) -> None:
+    """Raise unless the shapes fit (decided by the caller) and the tensors are dense, of one supported dtype and on
+    one ROCm device: a kernel is given pointers and counts its rows itself. (Alignment is the C entry's to check.)"""
+    if not fits or x.numel() >= x.shape[-1] << 31:
+        raise ValueError(f"{what}: shapes do not fit: {', '.join(str(tuple(t.shape)) for t in (x, *others))}")
+    dtype_code(x.dtype)
+    for t in (x, *others):
+        if t.dtype != x.dtype:
+            raise TypeError(f"{what}: operands must share one dtype")
+        if not t.is_contiguous() or t.device != x.device:
+            raise ValueError(f"{what}: operands must be contiguous and on one device")
+    _require_device(x)
+
+
+def _rows_of(x: torch.Tensor, width: int) -> bool:
+    return x.dim() >= 1 and x.shape[-1] == width > 0
+
+
+def _weight(w: torch.Tensor, x: torch.Tensor) -> bool:
+    return w.dim() == 2 and w.shape[0] > 0 and _rows_of(x, w.shape[1])
+
+
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """``weight * (x.float() * rsqrt(mean(x.float()^2) + eps)).to(dtype)`` in one launch."""
+    _check("rms_norm", weight.dim() == 1 and _rows_of(x, weight.shape[0]), x, weight)
     out = torch.empty_like(x)
     st = _native.load().mip_add_rms_norm(out.data_ptr(), None, x.data_ptr(), None, weight.data_ptr(),
                                          x.numel() // x.shape[-1], x.shape[-1], eps, _DTYPE_CODES[x.dtype],
@@ -78,6 +102,8 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
 def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
                  eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """``s = x + delta`` and the RMS norm of ``s``, in one launch; returns ``(s, normed)``."""
+    _check("add_rms_norm", weight.dim() == 1 and _rows_of(x, weight.shape[0]) and delta.shape == x.shape,
+           x, delta, weight)
     s, out = torch.empty_like(x), torch.empty_like(x)
     st = _native.load().mip_add_rms_norm(out.data_ptr(), s.data_ptr(), x.data_ptr(), delta.data_ptr(),
                                          weight.data_ptr(), x.numel() // x.shape[-1], x.shape[-1], eps,
@@ -113,6 +139,7 @@ def silu_mul_usable(gate_up: torch.Tensor) -> bool:
 
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` of the halves of the last dimension, in one launch."""
+    _check("silu_mul", gate_up.dim() >= 1 and gate_up.shape[-1] > 0 and gate_up.shape[-1] % 2 == 0, gate_up)
     inter = gate_up.shape[-1] // 2
     out = torch.empty((*gate_up.shape[:-1], inter), dtype=gate_up.dtype, device=gate_up.device)
     st = _native.load().mip_silu_mul(out.data_ptr(), gate_up.data_ptr(), gate_up.numel() // (2 * inter), inter,
@@ -173,6 +200,10 @@ def norm_linear(x: torch.Tensor, norm: torch.Tensor, eps: float, weight: torch.T
     With ``gate_up`` the weight holds gate rows, then as many up rows, and the result is
     ``silu(gate) * up``.
     """
+    extra = () if bias is None else (bias,)
+    _check("norm_linear", _weight(weight, x) and norm.shape == (x.shape[-1],)
+           and (bias is None or bias.shape == weight.shape[:1])
+           and not (gate_up and (extra or weight.shape[0] % 2)), x, weight, norm, *extra)
     n, k = weight.shape
     out = torch.empty((*x.shape[:-1], n // 2 if gate_up else n), dtype=x.dtype, device=x.device)
     st = _native.load().mip_norm_linear(out.data_ptr(), x.data_ptr(), norm.data_ptr(), eps, weight.data_ptr(),
@@ -194,6 +225,10 @@ def qkv_linear(x: torch.Tensor, norm: torch.Tensor | None, eps: float, weight: t
     """:func:`norm_linear` (of x itself where ``norm`` is None) with the rotary embedding applied to the first
     ``rot_heads`` heads of its output; cos, sin ``[B, 1, T, head_dim]``. The rotation is
     :func:`engine.paged_ops.rope_kv_append`'s, bit for bit."""
+    extra = tuple(t for t in (norm, bias) if t is not None)
+    _check("qkv_linear", _weight(weight, x) and x.dim() == 3 and (norm is None or norm.shape == (x.shape[-1],))
+           and (bias is None or bias.shape == weight.shape[:1]) and cos.dim() == 4
+           and cos.shape == sin.shape == (x.shape[0], 1, x.shape[1], cos.shape[-1]), x, weight, cos, sin, *extra)
     n, k = weight.shape
     d = cos.shape[-1]
     out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
@@ -208,6 +243,8 @@ def qkv_linear(x: torch.Tensor, norm: torch.Tensor | None, eps: float, weight: t
 
 def linear_residual(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
     """``residual + a @ weight.T`` in one launch."""
+    _check("linear_residual", _weight(weight, a) and residual.shape == (*a.shape[:-1], weight.shape[0]),
+           a, weight, residual)
     n, k = weight.shape
     out = torch.empty_like(residual)
     st = _native.load().mip_linear_residual(out.data_ptr(), a.data_ptr(), weight.data_ptr(), residual.data_ptr(),

@@ -45,3 +45,53 @@ def test_a_layer_whose_widths_disagree_is_left_to_torch(monkeypatch, wrong):
     assert layer._fusable(x)
     wrong(layer)
     assert not layer._fusable(x)
+
+
+def _bad_calls():
+    from engine import layer_ops as lo
+
+    def z(*shape, dtype=torch.bfloat16):
+        return torch.zeros(shape, dtype=dtype)
+
+    x, w, n = z(8, 1, 64), z(96, 64), z(64)
+    cs = z(8, 1, 1, 32)
+    return [
+        ("norm weight of another width", ValueError, lambda: lo.rms_norm(x, z(32), 1e-6)),
+        ("norm weight with two dimensions", ValueError, lambda: lo.rms_norm(x, z(1, 64), 1e-6)),
+        ("rows without elements", ValueError, lambda: lo.rms_norm(z(3, 0), z(0), 1e-6)),
+        ("delta of fewer rows", ValueError, lambda: lo.add_rms_norm(x, z(1, 1, 64), n, 1e-6)),
+        ("norm weight of another dtype", TypeError, lambda: lo.rms_norm(x, z(64, dtype=torch.float32), 1e-6)),
+        ("a dtype without kernels", TypeError, lambda: lo.rms_norm(x.double(), n.double(), 1e-6)),
+        ("strided rows", ValueError, lambda: lo.rms_norm(z(64, 8).t(), n, 1e-6)),
+        ("odd gate_up", ValueError, lambda: lo.silu_mul(z(4, 33))),
+        ("strided gate_up", ValueError, lambda: lo.silu_mul(z(4, 64)[:, :32])),
+        ("rows twice the weight's width", ValueError, lambda: lo.norm_linear(x, z(32), 1e-6, z(96, 32))),
+        ("norm of another width", ValueError, lambda: lo.norm_linear(x, z(32), 1e-6, w)),
+        ("short bias", ValueError, lambda: lo.norm_linear(x, n, 1e-6, w, z(48))),
+        ("bias beside gating", ValueError, lambda: lo.norm_linear(x, n, 1e-6, w, z(96), gate_up=True)),
+        ("rows twice the weight's width", ValueError, lambda: lo.qkv_linear(x, None, 0.0, z(96, 32), None, cs, cs, 3)),
+        ("tables of fewer rows", ValueError, lambda: lo.qkv_linear(x, n, 1e-6, w, None, cs[:1], cs[:1], 3)),
+        ("sin unlike cos", ValueError, lambda: lo.qkv_linear(x, n, 1e-6, w, None, cs, z(8, 1, 1, 16), 3)),
+        ("short bias", ValueError, lambda: lo.qkv_linear(x, n, 1e-6, w, z(64), cs, cs, 3)),
+        ("tables of another dtype", TypeError, lambda: lo.qkv_linear(x, n, 1e-6, w, None, cs.float(), cs.float(), 3)),
+        ("rows twice the weight's width", ValueError, lambda: lo.linear_residual(x, z(64, 32), x)),
+        ("residual of fewer rows", ValueError, lambda: lo.linear_residual(x, z(64, 64), x[:4])),
+        ("residual of another width", ValueError, lambda: lo.linear_residual(x, w, x)),
+        ("host tensors", RuntimeError, lambda: lo.linear_residual(x, z(64, 64), x)),
+        ("host tensors", RuntimeError, lambda: lo.silu_mul(z(4, 64))),
+    ]
+
+
+@pytest.mark.parametrize("i", range(23))
+def test_the_functions_refuse_operands_their_kernels_cannot_read(monkeypatch, i):
+    from engine import _native
+
+    def load():
+        raise AssertionError("a launch was reached")
+
+    monkeypatch.setattr(_native, "load", load)
+    calls = _bad_calls()
+    assert len(calls) == 23
+    what, error, call = calls[i]
+    with pytest.raises(error):
+        call()

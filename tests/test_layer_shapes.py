@@ -1,4 +1,4 @@
-"""Which layers and operands the fused layer kernels may be given: everything else is refused before a launch."""
+"""Which layers and operands the fused layer kernels and the step kernels may be given: the rest is refused on the host."""
 
 from __future__ import annotations
 
@@ -95,3 +95,24 @@ def test_the_functions_refuse_operands_their_kernels_cannot_read(monkeypatch, i)
     what, error, call = calls[i]
     with pytest.raises(error):
         call()
+
+
+@pytest.mark.parametrize("change", [
+    {"cu_q": [0, 3]}, {"cu_q": [[0, 3, 5]]}, {"cu_q": [0, 3, 5, 6]}, {"ctx_start": [[0, 0]]}, {"block_tables": [[0, 1]]},
+    {"block_tables": [0, 1]}, {"dtype": torch.int64}, {"strided": True}, {"n_tokens": -1}, {"max_q_len": -3},
+])
+def test_prefill_index_refuses_tensors_that_do_not_match(monkeypatch, change):
+    """cu_q holds one entry more than there are sequences, and every sequence has a table row."""
+    from engine import _native, paged_ops
+
+    def load():
+        raise AssertionError("a launch was reached")
+
+    monkeypatch.setattr(_native, "load", load)
+    dt = change.get("dtype", torch.int32)
+    cu, start, tab = (torch.tensor(change.get(n, d), dtype=dt) for n, d in (
+        ("cu_q", [0, 3, 5]), ("ctx_start", [0, 0]), ("block_tables", [[0, 1], [2, 3]])))
+    if change.get("strided"):
+        tab = tab.t()
+    with pytest.raises(ValueError):
+        paged_ops.prefill_index(cu, start, tab, change.get("n_tokens", 5), change.get("max_q_len", 3), 4)

@@ -32,14 +32,16 @@ __global__ __launch_bounds__(256) void step_rows_kernel(const int32_t* rows, int
 }
 
 // cos and sin of position * theta^(-2 j / D) for j < D / 2, both halves of a row alike. The steps and
-// their fp32 roundings are torch's (exponent, pow, reciprocal, angle, then cos and sin).
+// their fp32 roundings are torch's (exponent, pow, reciprocal, angle, then cos and sin), which divides
+// the exponent by D as a product with 1 / D: another value where D is no power of two.
 template <int DT>
 __global__ __launch_bounds__(256) void rope_tables_kernel(typename Elem<DT>::S* cos, typename Elem<DT>::S* sin,
                                                           const int64_t* positions, uint32_t total, uint32_t half,
                                                           float theta) {
+  const float inv_d = 1.0f / static_cast<float>(2 * half);
   for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < total; i += gridDim.x * 256u) {
     const uint32_t tok = i / half, j = i - tok * half;
-    const float e = static_cast<float>(j) * 2.0f / static_cast<float>(2 * half);
+    const float e = static_cast<float>(j) * 2.0f * inv_d;
     const float inv = 1.0f / powf(theta, e);
     const float ang = static_cast<float>(positions[tok]) * inv;
     const auto c = from_f32<DT>(cosf(ang)), s = from_f32<DT>(sinf(ang));

@@ -39,6 +39,20 @@ def test_rope_tables(gpu, dtype, d, theta):
         assert ((s2.double() - sin.double()).abs()[..., :half] <= 2 * bound).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [2, 6, 48, 64, 80, 96, 112, 128, 160, 192])
+def test_rope_tables_are_the_torch_steps_bit_for_bit(gpu, dtype, d):
+    """Head sizes that are no power of two too, where a quotient by d and a product with 1 / d differ."""
+    from engine.model import rope_cos_sin
+
+    announce(f"rope tables against torch {dtype} d={d}")
+    pos = torch.cat([torch.arange(2048, device=gpu), torch.randint(2048, 1 << 20, (512,), device=gpu)])[None]
+    for theta in (1e6, 1e4, 10000.1, 3):
+        cos, sin = rope_cos_sin(pos, d, theta, dtype)
+        c2, s2 = rope_cos_sin(torch.stack([pos, pos], dim=-1)[..., 0], d, theta, dtype)  # strided: torch's own ops
+        assert torch.equal(cos, c2) and torch.equal(sin, s2), theta
+
+
 @pytest.mark.parametrize("bs", [1, 16, 64])
 def test_decode_prepare(gpu, bs):
     from engine import paged_ops

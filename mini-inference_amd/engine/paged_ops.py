@@ -312,8 +312,9 @@ class _LayerCalls:
         return hit
 
     def _keep(self, kind: str, key: tuple, step, k_pool: torch.Tensor, v_pool: torch.Tensor, keep: tuple) -> None:
-        self._cached[kind] = (key, ctypes.addressof(step), k_pool.shape[0], k_pool.stride(0) * k_pool.element_size(),
-                              v_pool.stride(0) * v_pool.element_size(), step, keep)
+        self._cached[kind] = (key, ctypes.addressof(step), min(k_pool.shape[0], v_pool.shape[0]),
+                              k_pool.stride(0) * k_pool.element_size(), v_pool.stride(0) * v_pool.element_size(), step,
+                              keep)
 
 
 class DecodeStepCalls(_LayerCalls):

@@ -116,3 +116,15 @@ def test_prefill_index_refuses_tensors_that_do_not_match(monkeypatch, change):
         tab = tab.t()
     with pytest.raises(ValueError):
         paged_ops.prefill_index(cu, start, tab, change.get("n_tokens", 5), change.get("max_q_len", 3), 4)
+
+
+def test_a_kept_step_serves_only_layers_that_both_pools_hold():
+    """Later calls add the layer's offset to the pools' addresses: a layer that one of them lacks is checked in full."""
+    from engine import _native, paged_ops
+
+    calls = paged_ops._LayerCalls()
+    k, v = torch.zeros(4, 3, 2, 16, 8), torch.zeros(2, 3, 2, 16, 8)
+    calls._keep("decode", ("key",), _native.DecodeStep(), k, v, ())
+    assert calls._hit("decode", ("key",), 1) is not None
+    for layer in (2, 3, 4, -1, True, 1.0):
+        assert calls._hit("decode", ("key",), layer) is None

@@ -10,6 +10,7 @@ that its kernel cannot read.
 from __future__ import annotations
 
 import torch
+from torch.fx._symbolic_trace import is_fx_tracing as _is_fx_tracing
 
 from . import _native
 from .paged_ops import _DTYPE_CODES, _require_device, _stream_ptr, dtype_code
@@ -24,12 +25,13 @@ def _observed() -> bool:
     return (torch.compiler.is_compiling()  # first: a compiler that traces this function stops reading here
             or torch._C._len_torch_function_stack() > 0 or torch._C._len_torch_dispatch_stack() > 0
             or torch._C._functorch.peek_interpreter_stack() is not None or _FWD_AD._current_level >= 0
-            or torch._C._get_tracing_state() is not None or torch.is_autocast_enabled("cuda"))
+            or torch._C._get_tracing_state() is not None or _is_fx_tracing() or torch.is_autocast_enabled("cuda"))
 
 
 def _open(x: torch.Tensor) -> bool:
-    """Whether this device tensor's op may be taken over at all (asked before anything about its sizes)."""
-    return x.is_cuda and x.dtype in _DTYPE_CODES and not _observed()
+    """Whether this device tensor's op may be taken over at all (asked before anything about its sizes: a symbolic
+    tracer's stand-in for a tensor answers no such question)."""
+    return type(x) in _PLAIN and x.is_cuda and x.dtype in _DTYPE_CODES and not _observed()
 
 
 def _operands(x: torch.Tensor, *others: torch.Tensor) -> bool:
@@ -116,7 +118,7 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
 def rope_tables(positions: torch.Tensor, head_dim: int, theta: float,
                 dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor] | None:
     """cos/sin ``[B, 1, T, D]`` for ``positions [B, T]`` in one launch, or None where it does not apply."""
-    if (not positions.is_cuda or _observed() or type(positions) is not torch.Tensor or positions.dtype != torch.int64
+    if (type(positions) is not torch.Tensor or not positions.is_cuda or _observed() or positions.dtype != torch.int64
             or positions.dim() != 2 or not positions.is_contiguous() or dtype not in _DTYPE_CODES or head_dim % 2
             or type(theta) not in (float, int) or theta <= 0 or not 0 < positions.numel() * head_dim < 1 << 31
             or positions.device.index != torch.cuda.current_device()):

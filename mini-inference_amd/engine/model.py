@@ -194,6 +194,8 @@ class DecoderLayer(nn.Module):
 
     def _fusable(self, x: torch.Tensor) -> bool:
         """Whether the layer may run as its fused steps: unwatched submodules, operands the kernels take."""
+        if not layer_ops._open(x):
+            return False
         a, m, n1, n2 = self.attn, self.mlp, self.input_norm, self.post_attn_norm
         if not (_plain(n1, RMSNorm) and _plain(n2, RMSNorm) and _plain(a, Attention) and _plain(m, MLP)):
             return False

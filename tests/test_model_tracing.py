@@ -38,3 +38,54 @@ def test_modules_can_be_scripted_traced_and_compiled():
 @pytest.mark.skipif(not HAS_GPU, reason="no ROCm GPU in this environment")
 def test_modules_can_be_scripted_traced_and_compiled_on_the_gpu():
     _check("cuda")
+
+
+def _check_symbolic(dev):
+    """torch.fx: every module, and a model whose context is a constant, records the torch ops and gives their values."""
+    from engine.model import MLP, DecoderLayer, Qwen2Config, Qwen2ForCausalLM, RMSNorm, rope_cos_sin
+
+    cfg = Qwen2Config(vocab_size=64, hidden_size=64, intermediate_size=128, num_layers=2, num_heads=2, num_kv_heads=1,
+                      head_dim=32)
+
+    class Same:
+        def attend(self, layer_idx, q, k, v):
+            return q
+
+    class OfConstant(torch.nn.Module):  # the weights are symbols, the input is not
+        def __init__(self):
+            super().__init__()
+            self.norm, self.layer = RMSNorm(64, 1e-6), DecoderLayer(cfg, 0)
+            self.x = torch.randn(1, 5, 64, device=dev)
+            self.cos = torch.ones(1, 1, 5, 32, device=dev)
+
+        def forward(self, y):
+            return self.norm(self.x) + self.layer(self.x, self.cos, self.cos * 0, Same()) + y
+
+    class Whole(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.model = Qwen2ForCausalLM(cfg)
+
+        def forward(self, ids, pos):
+            return self.model(ids, pos, Same())
+
+    x = torch.randn(1, 5, 64, device=dev)
+    pos = torch.arange(5, device=dev)[None]
+    with torch.no_grad():
+        for mod, args in ((RMSNorm(64, 1e-6), (x,)), (MLP(cfg), (x,)), (OfConstant(), (x,)), (Whole(), (pos, pos))):
+            mod = mod.to(dev)
+            made = torch.fx.symbolic_trace(mod)
+            torch.testing.assert_close(made(*args), mod(*args), rtol=1e-5, atol=1e-5)
+        made = torch.fx.symbolic_trace(rope_cos_sin, concrete_args={"head_dim": 32, "theta": 1e6, "dtype": torch.float32})
+        for a, b in zip(made(pos, 32, 1e6, torch.float32), rope_cos_sin(pos, 32, 1e6, torch.float32)):
+            torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
+def test_modules_can_be_traced_symbolically():
+    _check_symbolic("cpu")
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not HAS_GPU, reason="no ROCm GPU in this environment")
+def test_modules_can_be_traced_symbolically_on_the_gpu():
+    _check_symbolic("cuda")

@@ -10,7 +10,9 @@ that its kernel cannot read.
 from __future__ import annotations
 
 import torch
+import torch.overrides
 from torch.fx._symbolic_trace import is_fx_tracing as _is_fx_tracing
+from torch.utils._device import DeviceContext
 
 from . import _native
 from .paged_ops import _DTYPE_CODES, _require_device, _stream_ptr, dtype_code
@@ -20,10 +22,17 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _MAX_ROW_BYTES = 32768
 
 
+def _function_mode() -> bool:
+    """Whether a mode sees torch calls. A default device (``torch.set_default_device``, ``with torch.device(..)``) is a
+    mode too, but one that only fills in the device of calls that name none."""
+    return torch._C._len_torch_function_stack() > 0 and any(
+        type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack())
+
+
 def _observed() -> bool:
     """Whether something other than the plain eager dispatch would see a torch op called now."""
     return (torch.compiler.is_compiling()  # first: a compiler that traces this function stops reading here
-            or torch._C._len_torch_function_stack() > 0 or torch._C._len_torch_dispatch_stack() > 0
+            or _function_mode() or torch._C._len_torch_dispatch_stack() > 0
             or torch._C._functorch.peek_interpreter_stack() is not None or _FWD_AD._current_level >= 0
             or torch._C._get_tracing_state() is not None or _is_fx_tracing() or torch.is_autocast_enabled("cuda"))
 

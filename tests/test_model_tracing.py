@@ -89,3 +89,64 @@ def test_modules_can_be_traced_symbolically():
 @pytest.mark.skipif(not HAS_GPU, reason="no ROCm GPU in this environment")
 def test_modules_can_be_traced_symbolically_on_the_gpu():
     _check_symbolic("cuda")
+
+
+def test_a_default_device_is_no_observer_and_other_modes_are():
+    """What the rule for the layer kernels takes for somebody watching the torch calls."""
+    from engine import layer_ops
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatched(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert not layer_ops._observed()
+    with torch.device("cpu"):
+        assert not layer_ops._observed()
+        with torch.device("meta"):
+            assert not layer_ops._observed()
+            with Seen():
+                assert layer_ops._observed()
+        with Dispatched():
+            assert layer_ops._observed()
+    torch.set_default_device("cpu")
+    try:
+        assert not layer_ops._observed()
+        with Seen():
+            assert layer_ops._observed()
+    finally:
+        torch.set_default_device(None)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not HAS_GPU, reason="no ROCm GPU in this environment")
+def test_layer_kernels_run_under_a_default_device(monkeypatch):
+    from engine import layer_ops
+    from engine.model import DecoderLayer, Qwen2Config, rope_cos_sin
+
+    cfg = Qwen2Config(vocab_size=64, hidden_size=64, intermediate_size=128, num_layers=1, num_heads=2, num_kv_heads=1,
+                      head_dim=32)
+
+    class Same:
+        def attend(self, layer_idx, q, k, v):
+            return q
+
+    layer = DecoderLayer(cfg, 0).to("cuda").requires_grad_(False)
+    x, pos = torch.randn(2, 3, 64, device="cuda"), torch.arange(3, device="cuda").repeat(2, 1)
+    calls = []
+    tables = layer_ops.rope_tables
+    monkeypatch.setattr(layer_ops, "rope_tables", lambda *a: calls.append(tables(*a)) or calls[-1])
+    with torch.inference_mode():
+        cos, sin = rope_cos_sin(pos, 32, 1e6, torch.float32)
+        want = layer(x, cos, sin, Same())
+        for dev in ("cuda", "cpu", "meta"):
+            with torch.device(dev):
+                assert layer._fusable(x)
+                cos, sin = rope_cos_sin(pos, 32, 1e6, torch.float32)
+                assert torch.equal(layer(x, cos, sin, Same()), want)
+    assert len(calls) == 4 and all(c is not None for c in calls)

@@ -180,12 +180,10 @@ __global__ __launch_bounds__(kNW * kWave) void paged_attn_f32(DecodeArgs a) {
     }
     f32_load_k<D>(kf, a, at, g);
     bool need = false;
-    bool sees[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int key = 4 * g + i;
-      sees[i] = ((valid >> key) & 1u) && base + key < lim;
-      s[i] = sees[i] ? s[i] * a.scale_log2 : -INFINITY;
+      s[i] = ((valid >> key) & 1u) && base + key < lim ? s[i] * a.scale_log2 : -INFINITY;
       need |= s[i] > m + kRescaleLog2;
     }
     if (__any(need)) {
@@ -202,7 +200,8 @@ __global__ __launch_bounds__(kNW * kWave) void paged_attn_f32(DecodeArgs a) {
     float p[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[i] = sees[i] ? fast_exp2(s[i] - m) : 0.f;
+      // A key that scores -inf weighs 0, also while nothing above it has been seen (m = -inf).
+      p[i] = s[i] == -INFINITY ? 0.f : fast_exp2(s[i] - m);
       l += p[i];
     }
     bool odd = false;  // an infinity or NaN in a value that not every row sees

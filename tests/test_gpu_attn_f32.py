@@ -119,3 +119,45 @@ def test_decode_agrees_with_the_valu_kernel(gpu):
         flat = torch.empty(q.numel() + 1, device=gpu)
         odd = flat[1:].view_as(q).copy_(q)
         assert torch.equal(paged_ops.paged_decode(odd, k, v, tab, ctx), got)
+
+
+def _minus_infinity(k, tab, spans, bs):
+    """Keys of sequence i at positions [a, b) score -inf for a query whose first element is positive."""
+    for i, spans_i in enumerate(spans):
+        for a, b in spans_i:
+            for pos in range(a, b):
+                k[int(tab[i, pos // bs]), :, pos % bs, 0] = -math.inf
+
+
+@pytest.mark.parametrize("algo", ["auto"])
+@pytest.mark.parametrize("d,hq,hkv,bs", [(64, 14, 2, 16), (128, 16, 2, 8), (64, 16, 1, 64)])
+def test_a_score_of_minus_infinity_weighs_nothing(gpu, algo, d, hq, hkv, bs):
+    """Whole tiles, wavefronts and partitions of keys that score -inf, before, between and after finite ones."""
+    from engine import _native, paged_ops
+
+    announce(f"fp32 scores of -inf d={d} hq={hq} bs={bs} {algo}")
+    lens = [100, 300, 520, 17, 64]
+    spans = [[(0, 64)], [(0, 256), (258, 300)], [(1, 519)], [(0, 16)], [(16, 64)]]
+    k, v, tab, gen = _pool(gpu, hkv, d, bs, lens, seed=d + bs)
+    _minus_infinity(k, tab, spans, bs)
+    q = torch.randn(len(lens), hq, d, generator=gen, device=gpu)
+    q[:, :, 0] = 1.0
+    ctx = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    prev = _native.set_decode_algo(algo)
+    got = paged_ops.paged_decode(q, k, v, tab, ctx)
+    _native.set_decode_algo(prev)
+    want = _exact(q, k, v, tab, [n - 1 for n in lens], [1] * len(lens), bs)
+    # d / 8 + sqrt(keys) roundings of the largest value, as for the finite cases.
+    bound = (d / 8 + 32) * 2.0 ** -24 * float(v.abs().max())
+    assert float((got.double() - want).abs().max()) <= bound
+    # The same keys under packed prefill: every row sees key 0, and the last ones more.
+    starts, lengths = [40, 0], [60, 33]
+    k, v, tab, gen = _pool(gpu, hkv, d, bs, [100, 33], seed=d)
+    _minus_infinity(k, tab, [[(1, 97)], [(1, 20)]], bs)
+    q = torch.randn(93, hq, d, generator=gen, device=gpu)
+    q[:, :, 0] = 1.0
+    cu = torch.tensor([0, 60, 93], dtype=torch.int32, device=gpu)
+    st = torch.tensor(starts, dtype=torch.int32, device=gpu)
+    got = paged_ops.paged_prefill(q, k, v, tab, cu, st, 60)
+    want = _exact(q, k, v, tab, starts, lengths, bs)
+    assert float((got.double() - want).abs().max()) <= bound

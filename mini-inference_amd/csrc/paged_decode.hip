@@ -263,7 +263,8 @@ __global__ __launch_bounds__(kNW * kWave) void paged_decode_part(DecodeArgs a) {
     float p[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      p[g] = f.kvalid ? fast_exp2(s[g] - m[g]) : 0.0f;
+      // A key that scores -inf weighs 0, also while nothing above it has been seen (m = -inf).
+      p[g] = s[g] == -INFINITY ? 0.0f : fast_exp2(s[g] - m[g]);
       l[g] += p[g];
     }
     if (c == 0) {

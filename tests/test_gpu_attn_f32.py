@@ -129,8 +129,8 @@ def _minus_infinity(k, tab, spans, bs):
                 k[int(tab[i, pos // bs]), :, pos % bs, 0] = -math.inf
 
 
-@pytest.mark.parametrize("algo", ["auto"])
-@pytest.mark.parametrize("d,hq,hkv,bs", [(64, 14, 2, 16), (128, 16, 2, 8), (64, 16, 1, 64)])
+@pytest.mark.parametrize("algo", ["auto", "valu"])
+@pytest.mark.parametrize("d,hq,hkv,bs", [(64, 14, 2, 16), (128, 16, 2, 8), (64, 16, 1, 64), (32, 3, 3, 16), (256, 4, 2, 1)])
 def test_a_score_of_minus_infinity_weighs_nothing(gpu, algo, d, hq, hkv, bs):
     """Whole tiles, wavefronts and partitions of keys that score -inf, before, between and after finite ones."""
     from engine import _native, paged_ops

@@ -188,7 +188,8 @@ class DecoderLayer(nn.Module):
 
     def forward(self, x, cos, sin, ctx):
         if self._fusable(x):
-            return self._fused(x, None, cos, sin, ctx, whole=True)[0]
+            x, delta = self._fused(x, None, cos, sin, ctx)
+            return x if delta is None else x + delta
         x = x + self.attn(self.input_norm(x), cos, sin, ctx)
         return x + self.mlp(self.post_attn_norm(x))
 
@@ -210,12 +211,12 @@ class DecoderLayer(nn.Module):
                 and n2.weight.shape == n1.weight.shape and layer_ops.norm_usable(n1.weight, x)
                 and layer_ops.usable(x, n2.weight, *w, *(() if bias is None else (bias,))))
 
-    def _fused(self, x, delta, cos, sin, ctx, whole=False):
+    def _fused(self, x, delta, cos, sin, ctx):
         """``forward`` of ``x + delta`` (None: of x), as ``(y, delta)`` whose sum it is (None: y is).
 
         Norms, bias, residual adds and gating run inside the linear layers where rows are few, and
         as one kernel each between library products where they are many; there the last residual
-        add is left to the caller, which has a norm to fuse it with, unless it asks for the ``whole``.
+        add is left to the caller, which may have a norm to fuse it with.
         """
         a, m, n1, n2 = self.attn, self.mlp, self.input_norm, self.post_attn_norm
         rows = x.shape[0] * x.shape[1]
@@ -253,9 +254,6 @@ class DecoderLayer(nn.Module):
         w = m.down_proj.weight
         if layer_ops.linear_residual_pays(rows, w) and layer_ops.usable(x, act):
             return layer_ops.linear_residual(act, w, x), None
-        if whole:  # x is this call's own by now: the product accumulates onto it
-            x.view(rows, -1).addmm_(act.reshape(rows, -1), w.t())
-            return x, None
         return x, F.linear(act, w)
 
 

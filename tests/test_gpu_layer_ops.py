@@ -335,3 +335,27 @@ def test_contexts_that_rotate_for_themselves_still_do(gpu):
         for a, b in zip(run(ctx, base), want):
             assert torch.equal(a, b)
     assert calls == ["sub", "wrap"]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@torch.inference_mode()
+def test_layers_called_one_by_one_give_the_models_bits(gpu, dtype):
+    """With many rows a layer hands its last residual add on; called by itself it rounds exactly as within the model."""
+    from engine.model import Qwen2Config, Qwen2ForCausalLM, rope_cos_sin
+
+    announce(f"layers one by one {dtype}")
+
+    class Same:
+        def attend(self, layer_idx, q, k, v):
+            return q
+
+    cfg = Qwen2Config(vocab_size=97, hidden_size=128, intermediate_size=320, num_layers=3, num_heads=4, num_kv_heads=2,
+                      head_dim=32)
+    model = Qwen2ForCausalLM(cfg).to(gpu).to(dtype).requires_grad_(False)
+    ids = torch.randint(0, 97, (1, 300), device=gpu)
+    pos = torch.arange(300, device=gpu)[None]
+    x = model.embed_tokens(ids)
+    cos, sin = rope_cos_sin(pos, 32, cfg.rope_theta, dtype)
+    for layer in model.layers:
+        x = layer(x, cos, sin, Same())
+    assert torch.equal(model.norm(x), model(ids, pos, Same()))

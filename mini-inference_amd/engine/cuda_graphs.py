@@ -26,6 +26,9 @@ partition kernels, whose grid grows with the longest table).
 
 from __future__ import annotations
 
+import gc
+import threading
+import weakref
 from collections.abc import Sequence
 
 import torch
@@ -47,11 +50,45 @@ def _kv_buckets(limit: int, step: int | None, block_size: int) -> list[int]:
     return sorted({-(-kv // block_size) * block_size for kv in raw})
 
 
+class _NoCollection:
+    """No cyclic garbage collection while any thread is inside.
+
+    A collection may destroy device objects that a reference cycle has kept (other graphs above
+    all), and their destructors synchronize, which ends the process while a stream is recording.
+    """
+
+    def __init__(self) -> None:
+        self._lock, self._depth, self._was_on = threading.Lock(), 0, False
+
+    def __enter__(self) -> None:
+        with self._lock:
+            if self._depth == 0:
+                self._was_on = gc.isenabled()
+                gc.disable()
+            self._depth += 1
+
+    def __exit__(self, *exc) -> None:
+        with self._lock:
+            self._depth -= 1
+            if self._depth == 0 and self._was_on:
+                gc.enable()
+
+
+_no_collection = _NoCollection()
+
+
 class _GraphDecodeContext:
-    """Attention for a captured decode step; reads everything from the static buffers."""
+    """Attention for a captured decode step; reads everything from the static buffers.
+
+    Its owner is held weakly: the owner holds the contexts, and a cycle would leave a dropped
+    decoder's graphs and buffers to the garbage collector. What a recorded graph reads is held
+    here (the model's weights, the static buffers, the scratch).
+    """
 
     def __init__(self, owner: "GraphedDecoder", batch: int, kv_len: int) -> None:
-        self.owner = owner
+        self._owner = weakref.ref(owner)
+        self.workspace = owner.workspace
+        self._reads = (owner.model, owner.device_tables, owner._inputs, owner.tables)
         self.cache = owner.cache
         self.batch, self.kv_len = batch, kv_len
         self.num_blocks = kv_len // owner.cache.block_size
@@ -70,6 +107,13 @@ class _GraphDecodeContext:
                                                   owner.cache.block_size, owner.cache.k.dtype,
                                                   max_blocks=self.num_blocks)[1]
 
+    @property
+    def owner(self) -> "GraphedDecoder":
+        owner = self._owner()
+        if owner is None:
+            raise ReferenceError("the GraphedDecoder of this context is gone")
+        return owner
+
     def prepare(self) -> None:
         """Inside the graph, once per step: table updates, the batch's rows, slot mapping, context lengths."""
         owner = self.owner
@@ -86,7 +130,7 @@ class _GraphDecodeContext:
         k_layer, v_layer = self.cache.k[layer_idx], self.cache.v[layer_idx]
         out = paged_ops.paged_decode_append(q[:, :, 0], k[:, :, 0], v[:, :, 0], k_layer, v_layer, self.slot_mapping,
                                             self.tables, self.context_lens, scale=self.scale,
-                                            max_blocks=self.num_blocks, workspace=self.owner.workspace,
+                                            max_blocks=self.num_blocks, workspace=self.workspace,
                                             plan=self.plan)
         return out.unsqueeze(2)
 
@@ -98,7 +142,7 @@ class _GraphDecodeContext:
         paged_ops.rope_kv_append(q1, k[:, :, 0], v[:, :, 0], cos[:, 0, 0], sin[:, 0, 0], k_layer, v_layer,
                                  self.slot_mapping)
         out = paged_ops.paged_decode(q1, k_layer, v_layer, self.tables, self.context_lens, scale=self.scale,
-                                     max_blocks=self.num_blocks, workspace=self.owner.workspace, plan=self.plan)
+                                     max_blocks=self.num_blocks, workspace=self.workspace, plan=self.plan)
         return out.unsqueeze(2)
 
 
@@ -162,9 +206,10 @@ class GraphedDecoder:
     def capture(self, batches: Sequence[int] | None = None) -> None:
         """Record one graph per (batch, kv length) bucket, largest first so smaller ones reuse its memory."""
         wanted = self.batch_buckets if batches is None else sorted({self._bucket(b) for b in batches})
-        for batch in reversed(wanted):
-            for kv_len in reversed(self.kv_buckets):
-                self._capture_one(batch, kv_len)
+        with _no_collection:
+            for batch in reversed(wanted):
+                for kv_len in reversed(self.kv_buckets):
+                    self._capture_one(batch, kv_len)
         torch.cuda.synchronize()
 
     def _bucket(self, n: int) -> int:

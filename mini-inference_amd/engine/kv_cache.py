@@ -493,6 +493,10 @@ class PagedDecodeContext:
             self.cache.lengths[s] += 1
 
 
+# What PackedPrefillContext's layer calls are bound to: assigning one of these rebinds them.
+_PREFILL_STEP = frozenset(("cache", "block_tables", "cu_q", "ctx_start", "slot_mapping", "max_q_len"))
+
+
 class PackedPrefillContext:
     """Several prompts packed end to end in one forward pass (engine/kv_cache.py:218-301).
 
@@ -553,13 +557,25 @@ class PackedPrefillContext:
         self._mask_built = False
         self._mask = None
         self._read_at = None
+        self._write_at: tuple[torch.Tensor, torch.Tensor] | None = None
         self._calls: paged_ops.PrefillStepCalls | None = None
+
+    def __setattr__(self, name: str, value) -> None:
+        object.__setattr__(self, name, value)
+        if name in _PREFILL_STEP:  # the layer calls are laid out for the tensors they were given
+            object.__setattr__(self, "_calls", None)
 
     @property
     def write_at(self) -> tuple[torch.Tensor, torch.Tensor]:
-        """``(block, offset)`` of each new token (engine/kv_cache.py:247), from ``slot_mapping``."""
-        bs = self.cache.block_size
-        return torch.div(self.slot_mapping, bs, rounding_mode="floor"), self.slot_mapping % bs
+        """``(block, offset)`` of each new token (engine/kv_cache.py:247), from ``slot_mapping`` unless set."""
+        if self._write_at is None:
+            bs = self.cache.block_size
+            self._write_at = torch.div(self.slot_mapping, bs, rounding_mode="floor"), self.slot_mapping % bs
+        return self._write_at
+
+    @write_at.setter
+    def write_at(self, value: tuple[torch.Tensor, torch.Tensor]) -> None:
+        self._write_at = value
 
     def _build_mask(self) -> None:
         """The reference's mask and read-back index (engine/kv_cache.py:262-279), built on demand."""

@@ -266,7 +266,7 @@ def prepare_paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
             k_cache.data_ptr(), v_cache.data_ptr(), nb, block_tables.data_ptr(), block_tables.stride(0),
             context_lens.data_ptr(), b, hq, hkv, d, bs, mb, scale, ws_ptr, ws_bytes, plan_ptr, plan_bytes, code,
             _stream_ptr(q.device))
-    keep = (out, q, k_cache, v_cache, block_tables, context_lens, workspace, plan)
+    keep = (out, q, k_cache, v_cache, block_tables, context_lens, workspace, plan)  # [4:8]: the step's
     if append is None:
         return PreparedCall(lib.mip_paged_decode, args, "mip_paged_decode", keep), out
     k, v, slot_mapping = append
@@ -312,6 +312,7 @@ class _LayerCalls:
         return hit
 
     def _keep(self, kind: str, key: tuple, step, k_pool: torch.Tensor, v_pool: torch.Tensor, keep: tuple) -> None:
+        # keep: the tensors that the struct points to, and none of a layer's own.
         self._cached[kind] = (key, ctypes.addressof(step), min(k_pool.shape[0], v_pool.shape[0]),
                               k_pool.stride(0) * k_pool.element_size(), v_pool.stride(0) * v_pool.element_size(), step,
                               keep)
@@ -349,7 +350,8 @@ class DecodeStepCalls(_LayerCalls):
         call()
         if call is not _noop and q.shape[2] == k.shape[2] == v.shape[2] == 1:
             a = call._args
-            self._keep("append", key, self._struct(a[7:], a[2:6], a[6]), k_pool, v_pool, call.keep)
+            self._keep("append", key, self._struct(a[7:], a[2:6], a[6]), k_pool, v_pool,
+                       (self.slot_mapping, *call.keep[4:8]))
         return out.unsqueeze(2)
 
     def attend(self, layer: int, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor) -> torch.Tensor:
@@ -370,7 +372,7 @@ class DecodeStepCalls(_LayerCalls):
                                          self.scale, None, self.max_blocks, plan=self._plan(q1.shape[1], q1.dtype))
         call()
         if call is not _noop and q.shape[2] == 1:
-            self._keep("decode", key, self._struct(call._args, (0, 0, 0, 0), None), k_pool, v_pool, call.keep)
+            self._keep("decode", key, self._struct(call._args, (0, 0, 0, 0), None), k_pool, v_pool, call.keep[4:8])
         return out.unsqueeze(2)
 
     @staticmethod
@@ -389,7 +391,7 @@ class DecodeStepCalls(_LayerCalls):
                                       v_pool[layer], self.slot_mapping)
         call()
         if call is not _noop and all(t.shape[2] == 1 for t in (q, k, v)):
-            self._keep("rope", key, _rope_struct(call._args), k_pool, v_pool, call.keep)
+            self._keep("rope", key, _rope_struct(call._args), k_pool, v_pool, (self.slot_mapping,))
 
 
 def _rope_hit(calls: _LayerCalls, layer, key, q, k, v, cos, sin, k_pool, v_pool) -> bool:
@@ -439,7 +441,7 @@ class PrefillStepCalls(_LayerCalls):
             step = _native.PrefillStep(k_stride_tok=a[2], k_stride_head=a[3], v_stride_tok=a[4], v_stride_head=a[5],
                                        slot_mapping=a[9], num_cache_blocks=a[8], n_tokens=a[10], num_kv_heads=a[11],
                                        head_dim=a[12], block_size=a[13], dtype=a[14])
-            self._keep("append", key, step, k_pool, v_pool, call.keep)
+            self._keep("append", key, step, k_pool, v_pool, (self.slot_mapping,))
 
     def rope_append(self, layer: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor,
                     sin: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor) -> None:
@@ -451,7 +453,7 @@ class PrefillStepCalls(_LayerCalls):
                                       sin[0, 0], k_pool[layer], v_pool[layer], self.slot_mapping)
         call()
         if call is not _noop and all(t.shape[0] == 1 for t in (q, k, v)):
-            self._keep("rope", key, _rope_struct(call._args), k_pool, v_pool, call.keep)
+            self._keep("rope", key, _rope_struct(call._args), k_pool, v_pool, (self.slot_mapping,))
 
     def attend(self, layer: int, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor) -> torch.Tensor:
         """:func:`paged_prefill` of one layer; returns ``[1, Hq, N, D]``, a view of ``[N, Hq, D]``."""
@@ -478,7 +480,7 @@ class PrefillStepCalls(_LayerCalls):
                                        ctx_start=a[12], num_seqs=a[13], max_q_len=a[14], num_heads=a[15],
                                        num_kv_heads=a[16], head_dim=a[17], block_size=a[18], max_blocks_per_seq=a[19],
                                        scale=a[20], dtype=a[21])
-            self._keep("attend", key, step, k_pool, v_pool, call.keep)
+            self._keep("attend", key, step, k_pool, v_pool, (self.block_tables, self.cu_q, self.ctx_start))
         return out.transpose(0, 1).unsqueeze(0)
 
 

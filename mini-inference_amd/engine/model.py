@@ -78,14 +78,16 @@ class AttentionContext(Protocol):
 
 
 def _plain(module: nn.Module, cls: type) -> bool:
-    """Whether calling ``module`` does what ``cls.forward`` says and nothing else: its exact class, no hooks.
+    """Whether calling ``module`` does what this file's (or torch's) ``cls.forward`` says and nothing else: its exact
+    class, unpatched, uncompiled, no hooks.
 
     A fused step that passes a submodule's call by is only taken where nobody watches that call.
     """
     if torch.compiler.is_compiling():
         return False
     g = nn.modules.module
-    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
+    return (type(module) is cls and cls.forward is _FORWARD[cls] and "forward" not in module.__dict__
+            and module._compiled_call_impl is None and not module._forward_hooks
             and not module._forward_pre_hooks and not module._backward_hooks and not module._backward_pre_hooks
             and not g._global_forward_hooks and not g._global_forward_pre_hooks and not g._global_backward_hooks
             and not g._global_backward_pre_hooks)
@@ -255,6 +257,9 @@ class DecoderLayer(nn.Module):
         if layer_ops.linear_residual_pays(rows, w) and layer_ops.usable(x, act):
             return layer_ops.linear_residual(act, w, x), None
         return x, F.linear(act, w)
+
+
+_FORWARD = {cls: cls.forward for cls in (nn.Linear, RMSNorm, Attention, MLP, DecoderLayer)}
 
 
 class Qwen2ForCausalLM(nn.Module):

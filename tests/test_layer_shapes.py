@@ -47,6 +47,26 @@ def test_a_layer_whose_widths_disagree_is_left_to_torch(monkeypatch, wrong):
     assert not layer._fusable(x)
 
 
+def test_a_submodule_whose_call_means_something_else_is_called(monkeypatch):
+    """Another forward, on the class or on the object, a hook or a compiled call: the fused steps pass none of them by."""
+    from engine import layer_ops
+    from engine.model import MLP, Attention, RMSNorm
+
+    monkeypatch.setattr(layer_ops, "_open", lambda x: True)
+    monkeypatch.setattr(layer_ops, "_operands", lambda x, *others: True)
+    x = torch.zeros(8, 1, 64)
+    for cls in (RMSNorm, Attention, MLP, nn.Linear):
+        with monkeypatch.context() as m:
+            m.setattr(cls, "forward", lambda self, *args: args[0])
+            assert not _layer()._fusable(x)
+    for change in (lambda m: setattr(m.mlp, "forward", lambda y: y), lambda m: m.attn.o_proj.compile(backend="eager"),
+                   lambda m: m.input_norm.register_forward_pre_hook(lambda *a: None)):
+        layer = _layer()
+        assert layer._fusable(x)
+        change(layer)
+        assert not layer._fusable(x)
+
+
 def _bad_calls():
     from engine import layer_ops as lo
 

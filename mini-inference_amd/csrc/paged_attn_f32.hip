@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kNW * kWave) void paged_attn_f32(DecodeArgs a) {
   // Keys below this are seen by every row.
   const int all_see = min(first + r0 / a.group, cap);
 
-  float m = -INFINITY, l = 0.f;
+  float m = kNoScore, l = 0.f;
   f32x4_t acc[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kNW * kWave) void paged_attn_f32(DecodeArgs a) {
       mx = fmaxf(mx, __shfl_xor(mx, 16));
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       const float mn = fmaxf(m, mx);
-      const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - mn);
+      const float alpha = fast_exp2(m - mn);
       l *= alpha;
 #pragma unroll
       for (int t = 0; t < T; ++t) acc[t] *= alpha;
@@ -200,8 +200,7 @@ __global__ __launch_bounds__(kNW * kWave) void paged_attn_f32(DecodeArgs a) {
     float p[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      // A key that scores -inf weighs 0, also while nothing above it has been seen (m = -inf).
-      p[i] = s[i] == -INFINITY ? 0.f : fast_exp2(s[i] - m);
+      p[i] = fast_exp2(s[i] - m);  // 0 for a key that is not seen, or scores -inf: m is finite
       l += p[i];
     }
     bool odd = false;  // an infinity or NaN in a value that not every row sees
@@ -272,9 +271,7 @@ __global__ __launch_bounds__(kNW * kWave) void paged_attn_f32(DecodeArgs a) {
     float A = 0.f, Ls = 0.f;
 #pragma unroll
     for (int ww = 0; ww < kNW; ++ww) {
-      const float mw = sh_m[ww][r];
-      const float wt = mw == -INFINITY ? 0.f : fast_exp2(mw - mx);
-      // A wavefront without keys for the row has weight 0 and sums of 0.
+      const float wt = fast_exp2(sh_m[ww][r] - mx);  // a wavefront without keys for the row has sums of 0
       A = fmaf(wt, sh_acc[ww][r][d], A);
       Ls = fmaf(wt, sh_l[ww][r], Ls);
     }

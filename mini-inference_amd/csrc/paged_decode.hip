@@ -212,7 +212,7 @@ __global__ __launch_bounds__(kNW * kWave) void paged_decode_part(DecodeArgs a) {
   float m[G], l[G], acc[G][VEPL];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    m[g] = -INFINITY;
+    m[g] = kNoScore;
     l[g] = 0.0f;
 #pragma unroll
     for (int e = 0; e < VEPL; ++e) acc[g][e] = 0.0f;
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(kNW * kWave) void paged_decode_part(DecodeArgs a) {
 #pragma unroll
         for (int o = LPR; o < kWave; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
         const float mn = fmaxf(m[g], mx);
-        const float alpha = (m[g] == -INFINITY) ? 0.0f : fast_exp2(m[g] - mn);
+        const float alpha = fast_exp2(m[g] - mn);
         l[g] *= alpha;
 #pragma unroll
         for (int e = 0; e < VEPL; ++e) acc[g][e] *= alpha;
@@ -263,8 +263,7 @@ __global__ __launch_bounds__(kNW * kWave) void paged_decode_part(DecodeArgs a) {
     float p[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      // A key that scores -inf weighs 0, also while nothing above it has been seen (m = -inf).
-      p[g] = s[g] == -INFINITY ? 0.0f : fast_exp2(s[g] - m[g]);
+      p[g] = fast_exp2(s[g] - m[g]);  // 0 for a key that is none, or scores -inf: m is finite
       l[g] += p[g];
     }
     if (c == 0) {
@@ -361,8 +360,7 @@ __global__ __launch_bounds__(kNW * kWave) void paged_decode_part(DecodeArgs a) {
     float A = 0.0f, Ls = 0.0f;
 #pragma unroll
     for (int ww = 0; ww < kNW; ++ww) {
-      const float mw = sh_m[ww][g];
-      const float wt = (mw == -INFINITY) ? 0.0f : fast_exp2(mw - mx);
+      const float wt = fast_exp2(sh_m[ww][g] - mx);  // a wavefront without keys has sums of 0
       A = fmaf(wt, sh_acc[ww][g][d], A);
       Ls = fmaf(wt, sh_l[ww][g], Ls);
     }

@@ -11,6 +11,10 @@ namespace decode {
 constexpr int kNW = 4;                  // wavefronts per workgroup
 constexpr float kRescaleLog2 = 8.0f;    // lazy-rescale threshold, log2 units (p <= 256)
 
+// The running maximum of the fp32-score kernels before any key: the lowest finite value, so that a
+// difference with a score of -inf is -inf (weight 0) and never -inf - -inf.
+constexpr float kNoScore = -3.4028234663852886e38f;
+
 struct DecodeArgs {
   char* out;
   int64_t out_sb, out_sh;  // elements

@@ -18,12 +18,14 @@
 // What bounds it: at the short contexts that fp32 runs have, the chain of memory round trips
 // (lengths, table, keys, merge) and each wavefront's steps; at long prefills the fp32 matrix rate
 // (157 TFLOP/s). Against the VALU kernel, which reduced every score across lanes, took 8 keys a
-// step and gave each new token a workgroup of its own (graph replay, 14q/2kv d64 | 28q/4kv d128):
+// step and gave each new token a workgroup of its own (graph replay, 14q/2kv d64 | 28q/4kv d128; the
+// rules that choose between the two lie in paged_decode.hip, with the other group sizes):
 //   decode, 8 sequences of 16-256 keys 16.5 -> 8.4 | 21.7 -> 12.9 us; 64 of 2,000 44.4 -> 37.1 | 130 -> 130
 //   prefill, 8 prompts of 16-256       38.5 -> 20.0 | 104 -> 58.3;   8 of 1,024 740 -> 245 | 2811 -> 961
-// The sums are kept at least as exact as the VALU kernel's (a score in chains of 8 products, a
-// tile's values pairwise; relative error against 64 bits over 500-1,024 keys 2.1e-7 -> 1.7e-7),
-// which costs 5-15 %: single chains took 7.4 and 18.8 us on the two 14q/2kv mixes, at 2.9e-7.
+// The sums are kept at least as exact as the VALU kernel's: a score in chains of 8 products, a tile's
+// values pairwise. Decode, relative error against 64 bits at both head sizes, 64 sequences x 8 seeds:
+// 7.9-8.0e-8 over 1-16 keys (0.99 of the VALU kernel's), 1.3e-7 over 16-64 (0.97), 1.4e-7 over 16-256 (0.89),
+// 1.7e-7 over 500-1,024 (0.80), 1.9e-7 over 1,000-4,096 (0.83). That costs 5-15 %: single chains took 7.4 and 18.8 us on the two 14q/2kv mixes, at 2.9e-7.
 // 8 wavefronts per workgroup: 7.2 / 39.5 us (decode), 25.0 / 302 (prefill); two row tiles per
 // wavefront: 20.8 / 231 | 79.1 / 996 (prefill; a workgroup's steps get twice as long), single chains.
 #include "paged_decode_common.h"

@@ -678,6 +678,19 @@ bool mfma_eligible(int dtype, int d, int g) {
 
 bool f32_eligible(int dtype, int d, int g) { return dtype == MIP_F32 && (d == 64 || d == 128) && g >= 1 && g <= 16; }
 
+// Where the fp32 matrix-core kernel decodes faster than the VALU kernel (by the shape alone, so that a
+// sequence's result does not depend on what else is in the step). Its tile has 16 rows whatever the
+// group holds, so its time hardly grows with the group and the VALU kernel's does. Graph replay, us,
+// matrix-core / VALU, 8 sequences of 16-256 keys | 64 of 2,000 | 128 of 200, 4 kv heads:
+//   head_dim 64:  g 1 7.7/7.6 | 45.4/44.4 | -     g 2 7.7/8.4 | 46.6/47.3 | 13.0/11.8   g 3 7.8/9.6 | 46.7/47.4 | 35.8/34.3
+//                 g 4 7.7/12.0 | 47.0/48.7 | 36.4/36.7     g 8 8.0/18.4 | 49.9/84.3 | -   (g 3, g 4: 16 kv heads for 128 of 200)
+//   head_dim 128: g 1 11.3/10.6 | 100/97 | -     g 4 11.7/18.0 | 111/104 | 83.5/81.2   g 6 11.9/20.3 | 119/116 | 22.6/21.6
+//                 g 7 12.2/22.0 | 125/129 | 40.2/43.2    g 8 12.4/32.8 | 125/163 | -
+// At head_dim 128 groups of 3 to 6 gain where sequences are few and short and lose 3 to 10 % on full
+// batches: they stay on the VALU kernel, which is never the slower one by more than the wait for a
+// handful of short sequences. (From 7 on it is the matrix-core kernel except below 16 keys: 5.8 / 5.0.)
+bool f32_decode_pays(int d, int g) { return g >= (d == 64 ? 4 : 7); }
+
 // Forced algorithm (mip_set_decode_algo; MIP_ALGO_AUTO = the default choice below). Its
 // first value comes from MIP_DECODE_ALGO=valu|mfma|stream, read once.
 int algo_from_env() {
@@ -693,14 +706,14 @@ std::atomic<int>& forced_algo() {
 // Default: the stream-K MFMA kernel for 16-bit data at head_dim 64/128 (balanced persistent
 // work split, the fastest under rocprof at the Qwen shapes) while its per-sequence scan fits
 // in LDS (batch <= 4096); otherwise the per-partition MFMA kernel; for fp32 at head_dim 64/128 the
-// fp32 MFMA kernel; the VALU kernel for the other head sizes and for groups of more than 16
-// heads. A forced algorithm applies where its kernel exists.
+// fp32 MFMA kernel where it pays; the VALU kernel for the rest. A forced algorithm applies where its
+// kernel exists.
 Algo choose_algo(int dtype, int d, int g, int batch) {
   const int f = forced_algo().load(std::memory_order_relaxed);
   const bool mfma_ok = mfma_eligible(dtype, d, g);
   const bool stream_ok = mfma_ok && stream_config(dtype, d, g, batch).ok;
   if (f == MIP_ALGO_VALU) return Algo::kValu;
-  if (f32_eligible(dtype, d, g)) return Algo::kF32;
+  if (f32_eligible(dtype, d, g) && (f == MIP_ALGO_MFMA || f32_decode_pays(d, g))) return Algo::kF32;
   if (f == MIP_ALGO_MFMA && mfma_ok) return Algo::kMfma;
   if (f == MIP_ALGO_STREAM && stream_ok) return Algo::kStream;
   return stream_ok ? Algo::kStream : mfma_ok ? Algo::kMfma : Algo::kValu;
@@ -851,31 +864,9 @@ KernelPair pick_mfma_d(int d, int g) {
   }
 }
 
-template <int D>
-KernelFn pick_f32_merge(int g) {
-  switch (g) {
-    case 1: return paged_decode_merge<MIP_F32, D, 1>;
-    case 2: return paged_decode_merge<MIP_F32, D, 2>;
-    case 3: return paged_decode_merge<MIP_F32, D, 3>;
-    case 4: return paged_decode_merge<MIP_F32, D, 4>;
-    case 5: return paged_decode_merge<MIP_F32, D, 5>;
-    case 6: return paged_decode_merge<MIP_F32, D, 6>;
-    case 7: return paged_decode_merge<MIP_F32, D, 7>;
-    case 8: return paged_decode_merge<MIP_F32, D, 8>;
-    case 9: return paged_decode_merge<MIP_F32, D, 9>;
-    case 10: return paged_decode_merge<MIP_F32, D, 10>;
-    case 11: return paged_decode_merge<MIP_F32, D, 11>;
-    case 12: return paged_decode_merge<MIP_F32, D, 12>;
-    case 13: return paged_decode_merge<MIP_F32, D, 13>;
-    case 14: return paged_decode_merge<MIP_F32, D, 14>;
-    case 15: return paged_decode_merge<MIP_F32, D, 15>;
-    case 16: return paged_decode_merge<MIP_F32, D, 16>;
-    default: return nullptr;
-  }
-}
-
 KernelPair pick_kernel(Algo algo, int dtype, int d, int g) {
-  if (algo == Algo::kF32) return {f32_decode_kernel(d), d == 64 ? pick_f32_merge<64>(g) : pick_f32_merge<128>(g)};
+  // The merge is the VALU kernel's, a group of more than 8 heads split over workgroups as there.
+  if (algo == Algo::kF32) return {f32_decode_kernel(d), pick_valu_d<MIP_F32>(d, valu_heads(g)).merge};
   if (algo == Algo::kMfma) {
     switch (dtype) {
       case MIP_F16: return pick_mfma_d<MIP_F16>(d, g);
@@ -894,6 +885,29 @@ KernelPair pick_kernel(Algo algo, int dtype, int d, int g) {
 }  // namespace
 
 namespace decode {
+namespace {
+
+// Where the fp32 matrix-core kernel runs a packed prefill faster than the VALU kernel, which has a
+// workgroup per (new token, kv head, up to 8 of its heads: h). `valu` and `tiles` are the workgroups of
+// each, `keys` the most a row can see.
+//   - Several tokens share a tile (valu >= 2 tiles), the VALU kernel takes more than one round of
+//     workgroups, and the keys it would read for each token are many, or its workgroups alone are.
+//     16 kv heads, one head each, head_dim 64 | 128, us, matrix-core / VALU: 64 tokens 5.9/7.0 | 9.0/7.7,
+//     100 7.0/10.5 | 10.8/11.3, 256 9.4/31 | 15.8/39; 16 prompts of 8 5.1/6.5 | 6.8/6.1, of 16 5.7/11.5 |
+//     8.3/11.5; 8 prompts of 512 118/629 | 244/816. One kv head: 256 tokens 9.0/8.3.
+//   - A row's chain is the longer one in the VALU kernel, which reduces each score over lanes for each
+//     of its h heads: the line lies where h^2 keys passes 16 head_dim. One prompt, us: h 2 200 tokens
+//     8.8/8.3 | 14.0/10.9, 256 9.1/9.2 | 14.6/12.6; h 4 32 5.5/4.9 | 8.0/5.6, 64 5.7/6.0 | 8.6/7.5, 100 6.8/8.0 |
+//     10.7/10.3; h 7 5 5.4/5.8 | 7.8/5.6, 32 5.6/6.3 | 8.2/7.0, 64 5.9/7.9 | 8.7/9.4; h 8 16 5.5/6.3 | 8.0/6.7, 32
+//     5.6/6.7 | 8.2/8.6. Where the tiles fill the chip and hold one token each, as decode.
+bool f32_prefill_pays(int d, int g, int64_t valu, int64_t tiles, int64_t keys) {
+  const bool shared = valu >= 2 * tiles;
+  if (shared && valu > 256 && (valu >= 32 * d || valu * keys >= (d == 64 ? 1 << 16 : 3 << 16))) return true;
+  const int64_t h = valu_heads(g);
+  return h * h * keys > 16 * d && (shared || tiles <= 256 || f32_decode_pays(d, g));
+}
+
+}  // namespace
 
 int valu_prefill_launch(void* out, int64_t out_stride_tok, int64_t out_stride_head, const void* q,
                         int64_t q_stride_tok, int64_t q_stride_head, const void* k_cache, const void* v_cache,
@@ -945,8 +959,11 @@ int valu_prefill_launch(void* out, int64_t out_stride_tok, int64_t out_stride_he
   a.max_q_len = max_q_len;
   a.gsplit = vsplit;
   a.group = group;
-  if (f32_eligible(dtype, head_dim, group) && static_cast<int64_t>(max_q_len) * group < (int64_t{1} << 30))
-    return f32_prefill_launch(a, num_seqs, head_dim, stream);
+  if (f32_eligible(dtype, head_dim, group) && static_cast<int64_t>(max_q_len) * group < (int64_t{1} << 30)) {
+    const int64_t tiles = (static_cast<int64_t>(max_q_len) * group + 15) / 16 * num_seqs * num_kv_heads;
+    if (f32_prefill_pays(head_dim, group, grid_x * num_kv_heads * vsplit, tiles, cap))
+      return f32_prefill_launch(a, num_seqs, head_dim, stream);
+  }
   hipLaunchKernelGGL(kp.part, dim3(static_cast<unsigned>(grid_x), num_kv_heads * vsplit, 1), dim3(kNW * kWave), 0,
                      stream, a);
   return status_from_hip(hipGetLastError());
@@ -993,7 +1010,7 @@ int paged_decode_impl(void* out, int64_t out_stride_b, int64_t out_stride_h, con
   if (!std::isfinite(scale)) return MIP_EINVAL;
   const int group = num_heads / num_kv_heads;
   const WsLayout wl = ws_layout(batch, num_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, dtype);
-  const int vsplit = wl.algo == Algo::kValu ? valu_split(group) : 1;
+  const int vsplit = wl.algo == Algo::kValu || wl.algo == Algo::kF32 ? valu_split(group) : 1;
   const KernelPair kp = pick_kernel(wl.algo == Algo::kStream ? Algo::kMfma : wl.algo, dtype, head_dim,
                                     wl.algo == Algo::kValu ? valu_heads(group) : group);
   if (!kp.part) return MIP_EUNSUPPORTED;
@@ -1080,7 +1097,8 @@ int paged_decode_impl(void* out, int64_t out_stride_b, int64_t out_stride_h, con
   if (static_cast<int64_t>(num_kv_heads) * vsplit > 65535) return MIP_EUNSUPPORTED;
   a.gsplit = vsplit;
   a.group = group;
-  hipLaunchKernelGGL(kp.part, dim3(wl.nparts, num_kv_heads * vsplit, batch), dim3(kNW * kWave), 0, s, a);
+  const int part_heads = wl.algo == Algo::kF32 ? num_kv_heads : num_kv_heads * vsplit;  // a tile holds the whole group
+  hipLaunchKernelGGL(kp.part, dim3(wl.nparts, part_heads, batch), dim3(kNW * kWave), 0, s, a);
   if (wl.nparts > 1) hipLaunchKernelGGL(kp.merge, dim3(num_kv_heads * vsplit, batch), dim3(256), 0, s, a);
   return status_from_hip(hipGetLastError());
 }

@@ -221,9 +221,9 @@ KernelFn f32_decode_kernel(int d);
 int f32_prefill_launch(const DecodeArgs& a, int num_seqs, int d, hipStream_t stream);
 
 // Packed prefill attention for the shapes the 16-bit MFMA prefill kernel does not cover: fp32 at
-// head_dim 64 / 128 and up to 16 query heads per kv head on the fp32 matrix-core kernel, other
-// head sizes (8 .. 256, powers of two) on the VALU decode kernel (paged_decode.hip). Arguments
-// as mip_paged_prefill, checked there.
+// head_dim 64 / 128 and up to 16 query heads per kv head on the fp32 matrix-core kernel where it
+// pays, the rest (head sizes 8 .. 256, powers of two) on the VALU decode kernel (paged_decode.hip).
+// Arguments as mip_paged_prefill, checked there.
 int valu_prefill_launch(void* out, int64_t out_stride_tok, int64_t out_stride_head, const void* q,
                         int64_t q_stride_tok, int64_t q_stride_head, const void* k_cache, const void* v_cache,
                         int64_t num_cache_blocks, const int32_t* block_tables, int64_t bt_stride, const int32_t* cu_q,

@@ -645,7 +645,7 @@ def paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     pool through ``block_tables`` (int32 ``[S, >= max_blocks]``). Returns ``out [N, Hq, D]``.
     Follows engine/kv_cache.py:268-294 (prefix read-back + mask) and :290-294 (packed causal).
     16-bit data at head_dim 64/128 runs the MFMA prefill kernel, fp32 at those sizes the fp32 MFMA
-    kernel (up to 16 query heads per kv head each), other shapes (power-of-two head sizes 8 to
+    kernel where it pays (up to 16 query heads per kv head each), other shapes (power-of-two head sizes 8 to
     256) the VALU kernel; anything else raises.
     """
     call, out = prepare_paged_prefill(q, k_cache, v_cache, block_tables, cu_q, ctx_start, max_q_len, scale, out,

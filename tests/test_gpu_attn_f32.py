@@ -50,9 +50,10 @@ def _exact(q, k, v, tab, starts, lengths, bs):
 
 
 # Groups around the 16-row tile, block sizes below, at and above the 16-key tile, token counts whose
-# (token, head) rows end inside, at and just past a 32-row tile, and a context of several rounds.
+# (token, head) rows end inside, at and just past a 16-row tile, and a context of several rounds. (One head
+# per kv head runs the matrix-core kernel from 8 kv heads on here, the VALU kernel below.)
 @pytest.mark.parametrize("d,hq,hkv,bs", [(64, 14, 2, 16), (64, 1, 1, 1), (64, 16, 1, 8), (64, 15, 1, 64), (128, 8, 2, 32),
-                                         (128, 4, 4, 16)])
+                                         (128, 4, 4, 16), (64, 8, 8, 4), (128, 8, 8, 16), (64, 16, 8, 32)])
 def test_prefill_tiles(gpu, d, hq, hkv, bs):
     from engine import paged_ops
 
@@ -161,3 +162,43 @@ def test_a_score_of_minus_infinity_weighs_nothing(gpu, algo, d, hq, hkv, bs):
     got = paged_ops.paged_prefill(q, k, v, tab, cu, st, 60)
     want = _exact(q, k, v, tab, starts, lengths, bs)
     assert float((got.double() - want).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("d,bs", [(64, 16), (128, 8)])
+@pytest.mark.parametrize("g", [1, 2, 3, 4, 6, 7, 8, 9, 15, 16])
+def test_decode_of_every_group_size(gpu, d, bs, g):
+    """The kernel that the group gets, and the matrix-core kernel where it is not that: one partition and several,
+    whose merge splits a group of more than 8."""
+    from engine import _native, paged_ops
+
+    lens = [1, 16, 17, 255, 256, 257, 700, 0]
+    k, v, tab, gen = _pool(gpu, 2, d, bs, lens, seed=d + g)
+    q = torch.randn(len(lens), 2 * g, d, generator=gen, device=gpu)
+    ctx = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    want = _exact(q[:-1], k, v, tab, [n - 1 for n in lens[:-1]], [1] * (len(lens) - 1), bs)
+    for algo in ("auto", "mfma", "valu"):
+        announce(f"fp32 decode d={d} group {g} {algo}")
+        prev = _native.set_decode_algo(algo)
+        got = paged_ops.paged_decode(q, k, v, tab, ctx)
+        _native.set_decode_algo(prev)
+        # d / 8 + sqrt(keys) roundings of the largest value.
+        assert float((got[:-1].double() - want).abs().max()) <= (d / 8 + 32) * 2.0 ** -24 * float(v.abs().max())
+        assert not got[-1].any()
+
+
+# Single prompts of one kv head with the table as wide as the prompt: the last length that the VALU kernel gets and the
+# first that the matrix-core kernel gets (h^2 keys > 16 d, h = heads per VALU workgroup), blocks of one key.
+@pytest.mark.parametrize("d,g,first", [(64, 2, 257), (64, 4, 65), (64, 8, 17), (64, 9, 41), (128, 4, 129), (128, 7, 42),
+                                       (128, 16, 33)])
+def test_prefill_on_both_sides_of_the_rule(gpu, d, g, first):
+    from engine import paged_ops
+
+    for n in (first - 1, first):
+        announce(f"fp32 prefill d={d} group {g} of {n} tokens")
+        k, v, tab, gen = _pool(gpu, 1, d, 1, [n], seed=n)
+        q = torch.randn(n, g, d, generator=gen, device=gpu)
+        cu = torch.tensor([0, n], dtype=torch.int32, device=gpu)
+        got = paged_ops.paged_prefill(q, k, v, tab, cu, cu[:1], n)
+        want = _exact(q, k, v, tab, [0], [n], 1)
+        # As in test_prefill_tiles, over at most 257 keys.
+        assert float((got.double() - want).abs().max()) <= (d + 257) / 8 * 2.0 ** -24 * float(v.abs().max())

@@ -688,7 +688,8 @@ bool f32_eligible(int dtype, int d, int g) { return dtype == MIP_F32 && (d == 64
 //                 g 7 12.2/22.0 | 125/129 | 40.2/43.2    g 8 12.4/32.8 | 125/163 | -
 // At head_dim 128 groups of 3 to 6 gain where sequences are few and short and lose 3 to 10 % on full
 // batches: they stay on the VALU kernel, which is never the slower one by more than the wait for a
-// handful of short sequences. (From 7 on it is the matrix-core kernel except below 16 keys: 5.8 / 5.0.)
+// handful of short sequences. (From 7 on it is the matrix-core kernel except over very few keys: 8 keys
+// 5.8 / 5.0, 30 keys in groups of 10 6.2 / 5.6.)
 bool f32_decode_pays(int d, int g) { return g >= (d == 64 ? 4 : 7); }
 
 // Forced algorithm (mip_set_decode_algo; MIP_ALGO_AUTO = the default choice below). Its

@@ -161,18 +161,30 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
 
 
 # Where the fused linear kernels beat the library's product and the separate kernels around it: a
-# workgroup reads its rows of the input again for every 16 to 64 weight rows, so they win while
-# the rows are few or the weight small. Lines between measured shapes (bf16, weights cold, graph
-# replay, us, fused against library), n x k by rows:
-#   norm + linear     1152 x 896: 4.5/8.6 at 8 rows, 5.7/11.2 at 64, 10.1/11.2 at 256;
-#                     2560 x 2048: 8.8/16.2 at 16, 13.2/16.6 at 65, 26.4/19.7 at 128;
-#                     2048 x 1536: 12.7/13.8 at 128, 15.5/14.6 at 256; 4608 x 3584: 20.0/16.4 at 8
-#   norm + gate + up  9728 x 896: 9.3/14.6 at 8, 16.3/18.3 at 64, 27.0/18.4 at 65;
-#                     17920 x 1536: 28.7/47.4 at 16, 35.7/26.1 at 32; 22016 x 2048: 37.4/52.4 at 16;
-#                     37888 x 3584: 104/65 at 8
-#   linear + residual 896 x 896: 3.8/8.5 at 8, 6.2/9.7 at 256; 896 x 4864: 10.5/20.3 at 8,
-#                     12.0/19.1 at 64, 17.8/15.5 at 96; 2048 x 2048: 11.7/13.8 at 64;
-#                     3584 x 3584: 10.9/15.1 at 16, 18.7/14.9 at 32; 3584 x 18944: 39.0/48.7 at 16
+# workgroup reads its rows of the input again for every 16 to 64 weight rows and K is split over its
+# wavefronts alone, so they win while the rows are few, the weight small and K short. Lines between
+# measured shapes (n x k by rows: fp16 | bf16, weights cold, graph replay, us, fused / library with the
+# same elementwise work; linear + residual with the RMS norm that follows on both sides):
+#   norm + linear     1152 x 896: 8 rows 4.2/7.7 | 4.5/8.7, 64 5.1/10.5 | 5.4/11.2, 256 9.9/10.4 | 10.2/11.3;
+#                     4096 x 2048: 16 9.4/14.6 | 9.6/16.7; 2048 x 4096: 16 14.5/14.6 | 14.8/18.9;
+#                     4608 x 3584: 8 - | 20.0/16.4; 2048 x 2048: 64 12.8/15.0 | 13.1/16.8;
+#                     1024 x 4096: 32 14.2/14.7 | 14.6/15.5, 33 19.3/14.2 | 20.0/17.9;
+#                     2048 x 1536: 96 12.6/12.4 | 12.9/13.8; 3072 x 1344: 65 18.9/16.6 | 19.5/18.0;
+#                     1536 x 1024: 256 10.1/11.2 | 10.3/12.0; 1024 x 1536: 129 13.7/10.3 | 14.1/11.8
+#   norm + gate + up  9728 x 896: 8 8.9/13.4 | 9.5/14.8, 64 16.1/17.0 | 16.6/18.5, 65 - | 27.0/18.4;
+#                     22016 x 2048: 16 36.7/50.1 | 37.6/52.3; 16384 x 3072: 1 33.2/28.3 | 34.6/29.4;
+#                     12288 x 1024: 17 20.4/17.8 | 20.2/19.2, 64 17.4/18.6 | 17.9/19.8;
+#                     8192 x 1536: 33 20.1/16.8 | 20.5/18.4
+#   linear + residual 896 x 896: 8 6.3/8.1 | 7.2/9.5, 256 9.2/10.5 | 10.0/11.8;
+#                     896 x 4864: 8 13.2/15.8 | 14.0/21.1, 64 15.0/15.6 | 15.8/21.4;
+#                     2048 x 2048: 64 15.5/15.9 | 17.4/18.6; 2048 x 2560: 33 16.4/13.5 | 18.5/16.3;
+#                     1536 x 1536: 32 9.4/11.1 | 11.1/13.2, 33 (384 workgroups) 12.8/10.6 | 14.4/13.3;
+#                     768 x 1344: 256 10.9/12.4 | 11.8/13.8; 512 x 2048: 256 12.2/10.7 | 12.9/11.5;
+#                     3584 x 18944: 1 31.0/52.3 | 32.0/53.5, 16 46.0/52.5 | 47.2/54.0;
+#                     5120 x 14336: 16 63.4/42.8 | 64.6/45.1
+# At up to 16 rows the library's time of linear + residual jumps with k: over n <= 4096 the fused kernel
+# is ahead for k up to 4864 and at 11008 and 18944, level at one row and behind at 8 to 16 rows for k =
+# 8192 (3584 x 8192, 16 rows: 21.4/19.3 | 22.2/20.7) and 14336 (36.5/30.7 | 37.5/31.5).
 _HALF = (torch.float16, torch.bfloat16)
 
 
@@ -182,26 +194,27 @@ def _linear_fits(rows: int, weight: torch.Tensor) -> bool:
 
 
 def norm_linear_pays(rows: int, weight: torch.Tensor) -> bool:
-    limit = 8 << 20 if rows <= 16 else 4 << 20 if rows <= 96 else 3 << 19
-    return _linear_fits(rows, weight) and weight.numel() <= limit
-
-
-def qkv_linear_pays(rows: int, weight: torch.Tensor, normed: bool) -> bool:
-    """As :func:`norm_linear_pays`, with the rotary kernel that the library's product leaves to be run (3 to 5 us);
-    ``normed``: x is normed already (1152 x 896 at 256 rows: 10.1 us with the rotation against 10.6 + 5.0, under
-    the profiler; 2048 x 1536 at 256 rows 12.9 against 9.9 + 5.0, not worth a rule of its own)."""
-    return norm_linear_pays(rows, weight) or (normed and _linear_fits(rows, weight) and weight.numel() <= 3 << 19)
+    """Also the rule of :func:`qkv_linear`, which besides saves the rotary kernel (3 to 5 us)."""
+    elements, k = ((8 << 20, 4096) if rows <= 16 else (4 << 20, 4096) if rows <= 32 else (4 << 20, 2048) if rows <= 64
+                   else (3 << 20, 2048) if rows <= 96 else (3 << 19, 1024))
+    return _linear_fits(rows, weight) and weight.numel() <= elements and weight.shape[1] <= k
 
 
 def norm_gate_up_pays(rows: int, weight: torch.Tensor) -> bool:
-    limit = 48 << 20 if rows <= 16 else 12 << 20 if rows <= 64 else 0
-    return _linear_fits(rows, weight) and weight.numel() <= limit
+    elements, k = ((48 << 20, 2048) if rows <= 16 else (9 << 20, 1024) if rows <= 32 else (12 << 20, 1152) if rows <= 64
+                   else (0, 0))
+    return _linear_fits(rows, weight) and weight.numel() <= elements and weight.shape[1] <= k
 
 
 def linear_residual_pays(rows: int, weight: torch.Tensor) -> bool:
     if not _linear_fits(rows, weight):
         return False
-    return rows <= 16 or weight.numel() <= (5 << 20 if rows <= 64 else 1 << 20)
+    n, k = weight.shape
+    if rows <= 16:
+        return n <= 4096 and k <= 20480  # one round of 16-column workgroups on 256 CUs
+    if rows <= 64:  # one round too; from n = 2048 on the tiles are 32 x 32
+        return n * k < 9 << 19 and (n >= 2048 or (rows + 15) // 16 * (n // 16) <= 256)
+    return n * k <= 1 << 20 and k <= 1536
 
 
 def norm_linear(x: torch.Tensor, norm: torch.Tensor, eps: float, weight: torch.Tensor, bias: torch.Tensor | None = None,

@@ -228,7 +228,7 @@ class DecoderLayer(nn.Module):
             x, normed = layer_ops.add_rms_norm(x, delta, n1.weight, n1.eps)
         # A context that takes rotated q and k in its fused append gets them from the projection itself.
         rotated = (getattr(ctx, "fuse_rope", False) and getattr(ctx, "takes_rotated", False)
-                   and layer_ops.qkv_linear_pays(rows, w, normed is not None)
+                   and layer_ops.norm_linear_pays(rows, w)
                    and layer_ops.rope_usable(cos, sin, x, c.head_dim))
         if rotated:
             src, norm = (x, n1.weight) if normed is None else (normed, None)

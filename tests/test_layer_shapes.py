@@ -148,3 +148,27 @@ def test_a_kept_step_serves_only_layers_that_both_pools_hold():
     assert calls._hit("decode", ("key",), 1) is not None
     for layer in (2, 3, 4, -1, True, 1.0):
         assert calls._hit("decode", ("key",), layer) is None
+
+
+@pytest.mark.parametrize("rule,rows,n,k,pays", [
+    ("norm_linear_pays", 8, 1152, 896, True), ("norm_linear_pays", 256, 1152, 896, True),
+    ("norm_linear_pays", 257, 1152, 896, False), ("norm_linear_pays", 16, 2048, 4096, True),
+    ("norm_linear_pays", 8, 4608, 3584, False), ("norm_linear_pays", 32, 1024, 4096, True),
+    ("norm_linear_pays", 33, 1024, 4096, False), ("norm_linear_pays", 64, 2048, 2048, True),
+    ("norm_linear_pays", 65, 3072, 1344, False), ("norm_linear_pays", 129, 1024, 1536, False),
+    ("norm_linear_pays", 8, 1160, 896, False), ("norm_linear_pays", 8, 1152, 900, False),
+    ("norm_gate_up_pays", 16, 22016, 2048, True), ("norm_gate_up_pays", 1, 16384, 3072, False),
+    ("norm_gate_up_pays", 64, 9728, 896, True), ("norm_gate_up_pays", 65, 9728, 896, False),
+    ("norm_gate_up_pays", 17, 12288, 1024, False), ("norm_gate_up_pays", 64, 12288, 1024, True),
+    ("norm_gate_up_pays", 33, 8192, 1536, False), ("linear_residual_pays", 16, 3584, 18944, True),
+    ("linear_residual_pays", 1, 5120, 14336, False), ("linear_residual_pays", 64, 896, 4864, True),
+    ("linear_residual_pays", 65, 896, 4864, False), ("linear_residual_pays", 33, 2048, 2560, False),
+    ("linear_residual_pays", 32, 1536, 1536, True), ("linear_residual_pays", 33, 1536, 1536, False),
+    ("linear_residual_pays", 256, 896, 896, True), ("linear_residual_pays", 256, 512, 2048, False),
+])
+def test_the_rules_take_the_shapes_that_were_measured_faster(rule, rows, n, k, pays):
+    from engine import layer_ops
+
+    for dtype in (torch.float16, torch.bfloat16):
+        assert getattr(layer_ops, rule)(rows, torch.empty(n, k, dtype=dtype, device="meta")) is pays
+    assert not getattr(layer_ops, rule)(rows, torch.empty(n, k, device="meta"))

@@ -266,9 +266,9 @@ def test_qkv_linear_rotates_as_the_rope_kernel(gpu, dtype, d, hq, hkv, k):
                                      pool.clone(), skip)
             return y.view(m, 1, n)
 
+        # The projection alone takes the same tiles as the one with the rotation: the same sums at every m.
         got = layer_ops.qkv_linear(x, norm, 1e-6, w, bias, cos, sin, hq + hkv)
-        if m <= 64:  # the same tiles, so the same sums
-            assert torch.equal(got, rotate(layer_ops.norm_linear(x, norm, 1e-6, w, bias)))
+        assert torch.equal(got, rotate(layer_ops.norm_linear(x, norm, 1e-6, w, bias)))
         # Of x as it is, and with no head rotated: the projection itself, rotated afterwards.
         plain = layer_ops.qkv_linear(x, None, 0.0, w, bias, cos, sin, 0)
         want = (x.double() @ w.double().t() + bias.double()).view(m, 1, n)
@@ -276,7 +276,13 @@ def test_qkv_linear_rotates_as_the_rope_kernel(gpu, dtype, d, hq, hkv, k):
         assert ((plain.double() - want).abs() <= 1.01 * U[dtype] * want.abs() + (k / 64 + 8) * 2 ** -24 * mag + TINY).all()
         assert torch.equal(layer_ops.qkv_linear(x, None, 0.0, w, bias, cos, sin, hq + hkv), rotate(plain))
         bare = layer_ops.qkv_linear(x, norm, 1e-6, w, None, cos, sin, hq + hkv)
-        assert torch.isfinite(bare.float()).all() and bare.shape == got.shape
+        assert torch.equal(bare, rotate(layer_ops.norm_linear(x, norm, 1e-6, w)))
+        # Norm and no rotation in the rotating kernel, against 64 bits (bounds as in test_small_linears).
+        h = norm64(x, norm, 1e-6)
+        want = h @ w.double().t() + bias.double()
+        spread = (h.square() @ w.double().square().t()).sqrt()
+        still = layer_ops.qkv_linear(x, norm, 1e-6, w, bias, cos, sin, 0)
+        assert ((still.double() - want).abs() <= 1.01 * U[dtype] * want.abs() + 8 * U[dtype] * spread + TINY).all()
 
 
 @torch.inference_mode()

@@ -65,11 +65,13 @@ def _row_ok(t: torch.Tensor, limit: int) -> bool:
     return nbytes % 16 == 0 and nbytes <= limit and t.numel() // t.shape[-1] < 1 << 31
 
 
+def _norm_fits(weight: torch.Tensor, x: torch.Tensor) -> bool:
+    return weight.dim() == 1 and x.dim() >= 1 and weight.shape[0] == x.shape[-1] and _row_ok(x, _MAX_ROW_BYTES)
+
+
 def norm_usable(weight: torch.Tensor, x: torch.Tensor, delta: torch.Tensor | None = None) -> bool:
     """Whether :func:`add_rms_norm` / :func:`rms_norm` take these (``delta`` of x's own shape)."""
-    if not _open(x):
-        return False
-    if weight.dim() != 1 or x.dim() < 1 or weight.shape[0] != x.shape[-1] or not _row_ok(x, _MAX_ROW_BYTES):
+    if not _open(x) or not _norm_fits(weight, x):
         return False
     if delta is None:
         return _operands(x, weight)
@@ -78,7 +80,10 @@ def norm_usable(weight: torch.Tensor, x: torch.Tensor, delta: torch.Tensor | Non
 
 def _check(what: str, fits: bool, x: torch.Tensor, *others: torch.Tensor) -> None:
     """Raise unless the shapes fit (decided by the caller) and the tensors are dense, of one supported dtype and on
-    one ROCm device: a kernel is given pointers and counts its rows itself. (Alignment is the C entry's to check.)"""
+    one ROCm device: a kernel is given pointers and counts its rows itself. (Alignment is the C entry's to check.)
+
+    Each function below has an underscored form without this check, for callers that have compared every shape and
+    asked ``usable`` (2 to 3 us a call, four calls a layer)."""
     if not fits or x.numel() >= x.shape[-1] << 31:
         raise ValueError(f"{what}: shapes do not fit: {', '.join(str(tuple(t.shape)) for t in (x, *others))}")
     dtype_code(x.dtype)
@@ -101,6 +106,10 @@ def _weight(w: torch.Tensor, x: torch.Tensor) -> bool:
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """``weight * (x.float() * rsqrt(mean(x.float()^2) + eps)).to(dtype)`` in one launch."""
     _check("rms_norm", weight.dim() == 1 and _rows_of(x, weight.shape[0]), x, weight)
+    return _rms_norm(x, weight, eps)
+
+
+def _rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     out = torch.empty_like(x)
     st = _native.load().mip_add_rms_norm(out.data_ptr(), None, x.data_ptr(), None, weight.data_ptr(),
                                          x.numel() // x.shape[-1], x.shape[-1], eps, _DTYPE_CODES[x.dtype],
@@ -115,6 +124,11 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
     """``s = x + delta`` and the RMS norm of ``s``, in one launch; returns ``(s, normed)``."""
     _check("add_rms_norm", weight.dim() == 1 and _rows_of(x, weight.shape[0]) and delta.shape == x.shape,
            x, delta, weight)
+    return _add_rms_norm(x, delta, weight, eps)
+
+
+def _add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
+                  eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     s, out = torch.empty_like(x), torch.empty_like(x)
     st = _native.load().mip_add_rms_norm(out.data_ptr(), s.data_ptr(), x.data_ptr(), delta.data_ptr(),
                                          weight.data_ptr(), x.numel() // x.shape[-1], x.shape[-1], eps,
@@ -151,6 +165,10 @@ def silu_mul_usable(gate_up: torch.Tensor) -> bool:
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` of the halves of the last dimension, in one launch."""
     _check("silu_mul", gate_up.dim() >= 1 and gate_up.shape[-1] > 0 and gate_up.shape[-1] % 2 == 0, gate_up)
+    return _silu_mul(gate_up)
+
+
+def _silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     inter = gate_up.shape[-1] // 2
     out = torch.empty((*gate_up.shape[:-1], inter), dtype=gate_up.dtype, device=gate_up.device)
     st = _native.load().mip_silu_mul(out.data_ptr(), gate_up.data_ptr(), gate_up.numel() // (2 * inter), inter,
@@ -228,6 +246,11 @@ def norm_linear(x: torch.Tensor, norm: torch.Tensor, eps: float, weight: torch.T
     _check("norm_linear", _weight(weight, x) and norm.shape == (x.shape[-1],)
            and (bias is None or bias.shape == weight.shape[:1])
            and not (gate_up and (extra or weight.shape[0] % 2)), x, weight, norm, *extra)
+    return _norm_linear(x, norm, eps, weight, bias, gate_up)
+
+
+def _norm_linear(x: torch.Tensor, norm: torch.Tensor, eps: float, weight: torch.Tensor,
+                 bias: torch.Tensor | None = None, gate_up: bool = False) -> torch.Tensor:
     n, k = weight.shape
     out = torch.empty((*x.shape[:-1], n // 2 if gate_up else n), dtype=x.dtype, device=x.device)
     st = _native.load().mip_norm_linear(out.data_ptr(), x.data_ptr(), norm.data_ptr(), eps, weight.data_ptr(),
@@ -240,8 +263,12 @@ def norm_linear(x: torch.Tensor, norm: torch.Tensor, eps: float, weight: torch.T
 
 def rope_usable(cos: torch.Tensor, sin: torch.Tensor, x: torch.Tensor, head_dim: int) -> bool:
     """Whether :func:`qkv_linear` can take these rotary tables for rows ``x [B, T, hidden]``."""
+    return _open(x) and _rope_fits(cos, sin, x, head_dim)
+
+
+def _rope_fits(cos: torch.Tensor, sin: torch.Tensor, x: torch.Tensor, head_dim: int) -> bool:
     return (cos.shape == sin.shape == (x.shape[0], 1, x.shape[1], head_dim) and head_dim % 16 == 0
-            and usable(x, cos, sin))
+            and _operands(x, cos, sin))
 
 
 def qkv_linear(x: torch.Tensor, norm: torch.Tensor | None, eps: float, weight: torch.Tensor, bias: torch.Tensor | None,
@@ -253,6 +280,11 @@ def qkv_linear(x: torch.Tensor, norm: torch.Tensor | None, eps: float, weight: t
     _check("qkv_linear", _weight(weight, x) and x.dim() == 3 and (norm is None or norm.shape == (x.shape[-1],))
            and (bias is None or bias.shape == weight.shape[:1]) and cos.dim() == 4
            and cos.shape == sin.shape == (x.shape[0], 1, x.shape[1], cos.shape[-1]), x, weight, cos, sin, *extra)
+    return _qkv_linear(x, norm, eps, weight, bias, cos, sin, rot_heads)
+
+
+def _qkv_linear(x: torch.Tensor, norm: torch.Tensor | None, eps: float, weight: torch.Tensor, bias: torch.Tensor | None,
+                cos: torch.Tensor, sin: torch.Tensor, rot_heads: int) -> torch.Tensor:
     n, k = weight.shape
     d = cos.shape[-1]
     out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
@@ -269,6 +301,10 @@ def linear_residual(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tenso
     """``residual + a @ weight.T`` in one launch."""
     _check("linear_residual", _weight(weight, a) and residual.shape == (*a.shape[:-1], weight.shape[0]),
            a, weight, residual)
+    return _linear_residual(a, weight, residual)
+
+
+def _linear_residual(a: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
     n, k = weight.shape
     out = torch.empty_like(residual)
     st = _native.load().mip_linear_residual(out.data_ptr(), a.data_ptr(), weight.data_ptr(), residual.data_ptr(),

@@ -104,7 +104,7 @@ class RMSNorm(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not torch.jit.is_scripting():
             if layer_ops.norm_usable(self.weight, x):
-                return layer_ops.rms_norm(x, self.weight, self.eps)
+                return layer_ops._rms_norm(x, self.weight, self.eps)
         xf = x.float()
         inv = torch.rsqrt(xf.square().mean(dim=-1, keepdim=True) + self.eps)
         return self.weight * (xf * inv).to(x.dtype)
@@ -175,7 +175,7 @@ class MLP(nn.Module):
     def gated(self, gate_up: torch.Tensor) -> torch.Tensor:
         if not torch.jit.is_scripting():
             if layer_ops.silu_mul_usable(gate_up):
-                return layer_ops.silu_mul(gate_up)
+                return layer_ops._silu_mul(gate_up)
         gate, up = gate_up.chunk(2, dim=-1)
         return F.silu(gate) * up
 
@@ -210,8 +210,8 @@ class DecoderLayer(nn.Module):
         # Every width: the kernels take a shape that torch would refuse for a longer list of rows.
         return (x.dim() == 3 and w[0].shape == (qkv, h) and w[1].shape == (h, c.q_size) and w[2].shape == (2 * inter, h)
                 and w[3].shape == (h, inter) and (bias is None or bias.shape == (qkv,))
-                and n2.weight.shape == n1.weight.shape and layer_ops.norm_usable(n1.weight, x)
-                and layer_ops.usable(x, n2.weight, *w, *(() if bias is None else (bias,))))
+                and n2.weight.shape == n1.weight.shape and layer_ops._norm_fits(n1.weight, x)
+                and layer_ops._operands(x, n1.weight, n2.weight, *w, *(() if bias is None else (bias,))))
 
     def _fused(self, x, delta, cos, sin, ctx):
         """``forward`` of ``x + delta`` (None: of x), as ``(y, delta)`` whose sum it is (None: y is).
@@ -225,37 +225,37 @@ class DecoderLayer(nn.Module):
         w, c = a.qkv_proj.weight, a.cfg
         normed = None
         if delta is not None:
-            x, normed = layer_ops.add_rms_norm(x, delta, n1.weight, n1.eps)
+            x, normed = layer_ops._add_rms_norm(x, delta, n1.weight, n1.eps)
         # A context that takes rotated q and k in its fused append gets them from the projection itself.
         rotated = (getattr(ctx, "fuse_rope", False) and getattr(ctx, "takes_rotated", False)
-                   and layer_ops.norm_linear_pays(rows, w)
-                   and layer_ops.rope_usable(cos, sin, x, c.head_dim))
+                   and layer_ops.norm_linear_pays(rows, w) and layer_ops._rope_fits(cos, sin, x, c.head_dim))
         if rotated:
             src, norm = (x, n1.weight) if normed is None else (normed, None)
-            qkv = layer_ops.qkv_linear(src, norm, n1.eps, w, a.qkv_proj.bias, cos, sin, c.num_heads + c.num_kv_heads)
+            qkv = layer_ops._qkv_linear(src, norm, n1.eps, w, a.qkv_proj.bias, cos, sin, c.num_heads + c.num_kv_heads)
         elif normed is not None:
             qkv = F.linear(normed, w, a.qkv_proj.bias)
         elif layer_ops.norm_linear_pays(rows, w):
-            qkv = layer_ops.norm_linear(x, n1.weight, n1.eps, w, a.qkv_proj.bias)
+            qkv = layer_ops._norm_linear(x, n1.weight, n1.eps, w, a.qkv_proj.bias)
         else:
-            qkv = F.linear(layer_ops.rms_norm(x, n1.weight, n1.eps), w, a.qkv_proj.bias)
+            qkv = F.linear(layer_ops._rms_norm(x, n1.weight, n1.eps), w, a.qkv_proj.bias)
         out, w = a.attend(qkv, cos, sin, ctx, rotated), a.o_proj.weight
-        if out.shape[:2] != x.shape[:2] or not layer_ops.usable(x, out):  # a context with outputs of its own kind
+        if out.shape != (*x.shape[:2], c.q_size) or not layer_ops._operands(x, out):  # outputs of the context's own kind
             x = x + F.linear(out, w)
             return x + m(n2(x)), None
         w2 = m.gate_up_proj.weight
         if layer_ops.linear_residual_pays(rows, w):
-            x = layer_ops.linear_residual(out, w, x)
-            normed = None if layer_ops.norm_gate_up_pays(rows, w2) else layer_ops.rms_norm(x, n2.weight, n2.eps)
+            x = layer_ops._linear_residual(out, w, x)
+            normed = None if layer_ops.norm_gate_up_pays(rows, w2) else layer_ops._rms_norm(x, n2.weight, n2.eps)
         else:
-            x, normed = layer_ops.add_rms_norm(x, F.linear(out, w), n2.weight, n2.eps)
+            x, normed = layer_ops._add_rms_norm(x, F.linear(out, w), n2.weight, n2.eps)
         if normed is None:
-            act = layer_ops.norm_linear(x, n2.weight, n2.eps, w2, gate_up=True)
+            act = layer_ops._norm_linear(x, n2.weight, n2.eps, w2, gate_up=True)
         else:
             act = m.gated(F.linear(normed, w2))
         w = m.down_proj.weight
-        if layer_ops.linear_residual_pays(rows, w) and layer_ops.usable(x, act):
-            return layer_ops.linear_residual(act, w, x), None
+        if (layer_ops.linear_residual_pays(rows, w) and act.shape == (*x.shape[:2], w.shape[1])
+                and layer_ops._operands(x, act)):
+            return layer_ops._linear_residual(act, w, x), None
         return x, F.linear(act, w)
 
 
@@ -285,7 +285,7 @@ class Qwen2ForCausalLM(nn.Module):
         if delta is None:
             return self.norm(x)
         if _plain(self.norm, RMSNorm) and layer_ops.norm_usable(self.norm.weight, x, delta):
-            return layer_ops.add_rms_norm(x, delta, self.norm.weight, self.norm.eps)[1]
+            return layer_ops._add_rms_norm(x, delta, self.norm.weight, self.norm.eps)[1]
         return self.norm(x + delta)
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:

@@ -378,6 +378,7 @@ class PagedDecodeContext:
     """
 
     fuse_rope = True
+
     def __init__(self, cache: PagedKVCache, slots: Sequence[int]) -> None:
         self.cache = cache
         self.slots = list(slots)
@@ -493,8 +494,20 @@ class PagedDecodeContext:
             self.cache.lengths[s] += 1
 
 
-# What PackedPrefillContext's layer calls are bound to: assigning one of these rebinds them.
-_PREFILL_STEP = frozenset(("cache", "block_tables", "cu_q", "ctx_start", "slot_mapping", "max_q_len"))
+def _step_input(name: str) -> property:
+    """An attribute that a prefill context's layer calls are laid out for: assigning it has them laid out again."""
+
+    def get(self):
+        try:
+            return self.__dict__[name]
+        except KeyError:
+            raise AttributeError(name) from None
+
+    def put(self, value) -> None:
+        self.__dict__[name] = value
+        self._calls = None
+
+    return property(get, put)
 
 
 class PackedPrefillContext:
@@ -509,6 +522,8 @@ class PackedPrefillContext:
     """
 
     fuse_rope = True
+    cache, block_tables, cu_q, ctx_start, slot_mapping, max_q_len = map(
+        _step_input, ("cache", "block_tables", "cu_q", "ctx_start", "slot_mapping", "max_q_len"))
 
     def __init__(self, cache: PagedKVCache, slots: Sequence[int], lengths: Sequence[int]) -> None:
         self.cache = cache
@@ -559,11 +574,6 @@ class PackedPrefillContext:
         self._read_at = None
         self._write_at: tuple[torch.Tensor, torch.Tensor] | None = None
         self._calls: paged_ops.PrefillStepCalls | None = None
-
-    def __setattr__(self, name: str, value) -> None:
-        object.__setattr__(self, name, value)
-        if name in _PREFILL_STEP:  # the layer calls are laid out for the tensors they were given
-            object.__setattr__(self, "_calls", None)
 
     @property
     def write_at(self) -> tuple[torch.Tensor, torch.Tensor]:

@@ -577,7 +577,7 @@ def prefill_index(cu_q: torch.Tensor, ctx_start: torch.Tensor, block_tables: tor
     ``last_index`` (int64 ``[S]``), from the tensors :func:`paged_prefill` takes. Follows
     engine/kv_cache.py:230-250, 562-573.
     """
-    if any(t.dtype != torch.int32 for t in (cu_q, ctx_start, block_tables)):
+    if not cu_q.dtype == ctx_start.dtype == block_tables.dtype == torch.int32:
         raise ValueError("cu_q, ctx_start and block_tables must be int32")
     if (ctx_start.dim() != 1 or cu_q.shape != (ctx_start.shape[0] + 1,) or block_tables.dim() != 2
             or block_tables.shape[0] < ctx_start.shape[0] or n_tokens < 0 or max_q_len < 0):

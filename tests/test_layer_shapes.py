@@ -172,3 +172,38 @@ def test_the_rules_take_the_shapes_that_were_measured_faster(rule, rows, n, k, p
     for dtype in (torch.float16, torch.bfloat16):
         assert getattr(layer_ops, rule)(rows, torch.empty(n, k, dtype=dtype, device="meta")) is pays
     assert not getattr(layer_ops, rule)(rows, torch.empty(n, k, device="meta"))
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_a_layer_whose_widths_disagree_raises_on_the_gpu_as_anywhere(gpu):
+    """torch's shape errors, before anything of the layer's own is launched out of range; a bias row broadcasts."""
+    class Same:
+        def attend(self, layer_idx, q, k, v):
+            return q
+
+    dt = torch.bfloat16
+    x = torch.randn(8, 1, 64, device=gpu).to(dt)
+    cs = torch.ones(8, 1, 1, 16, device=gpu, dtype=dt)
+
+    def run(change):
+        torch.manual_seed(0)
+        layer = _layer()
+        change(layer)
+        layer = layer.to(gpu, dt)
+        return layer._fusable(x), layer(x, cs, cs * 0, Same())
+
+    for bad in (lambda m: _resized(m.attn.o_proj, 64, 32), lambda m: _resized(m.attn.o_proj, 32, 64),
+                lambda m: _resized(m.attn.qkv_proj, 128, 64, bias=64), lambda m: _resized(m.mlp.down_proj, 64, 64)):
+        with pytest.raises(RuntimeError):
+            run(bad)
+    fused, want = run(lambda m: None)
+    assert fused
+
+    def row(m):
+        m.attn.qkv_proj.bias = nn.Parameter(m.attn.qkv_proj.bias[None], requires_grad=False)
+
+    fused, got = run(row)
+    assert not fused
+    # The same layer through torch's ops: each side rounds every intermediate once or twice.
+    assert float((got.double() - want.double()).norm() / want.double().norm()) <= 8 * 2.0 ** -8

@@ -23,7 +23,7 @@ from __future__ import annotations
 from collections import OrderedDict
 from collections.abc import Sequence
 from itertools import chain
-from operator import ge
+from operator import attrgetter, ge
 
 import numpy as np
 import torch
@@ -497,17 +497,11 @@ class PagedDecodeContext:
 def _step_input(name: str) -> property:
     """An attribute that a prefill context's layer calls are laid out for: assigning it has them laid out again."""
 
-    def get(self):
-        try:
-            return self.__dict__[name]
-        except KeyError:
-            raise AttributeError(name) from None
-
     def put(self, value) -> None:
-        self.__dict__[name] = value
+        setattr(self, "_" + name, value)
         self._calls = None
 
-    return property(get, put)
+    return property(attrgetter("_" + name), put)
 
 
 class PackedPrefillContext:
@@ -522,8 +516,8 @@ class PackedPrefillContext:
     """
 
     fuse_rope = True
-    cache, block_tables, cu_q, ctx_start, slot_mapping, max_q_len = map(
-        _step_input, ("cache", "block_tables", "cu_q", "ctx_start", "slot_mapping", "max_q_len"))
+    block_tables, cu_q, ctx_start, slot_mapping, max_q_len = map(
+        _step_input, ("block_tables", "cu_q", "ctx_start", "slot_mapping", "max_q_len"))
 
     def __init__(self, cache: PagedKVCache, slots: Sequence[int], lengths: Sequence[int]) -> None:
         self.cache = cache
@@ -540,7 +534,7 @@ class PackedPrefillContext:
         self.has_prefix = any(self.starts)
         self.ends = [a + n for a, n in zip(self.starts, self.lengths)]
         # Inputs of the paged prefill kernel: packed row offsets, cached lengths, tables.
-        self.max_q_len = max(self.lengths)
+        self._max_q_len = max(self.lengths)
         nb = max(1, cache.blocks_for(max(self.ends)))
         s_n = len(self.slots)
         host = torch.empty(2 * s_n + 1 + s_n * nb, dtype=torch.int32, pin_memory=dev.type == "cuda")
@@ -556,18 +550,18 @@ class PackedPrefillContext:
                                                               count=int(widths.sum()))
         n_tok = int(i32[s_n])
         on_dev = host.to(dev, non_blocking=True)
-        self.cu_q, self.ctx_start = on_dev[:s_n + 1], on_dev[s_n + 1:2 * s_n + 1]
-        self.block_tables = on_dev[2 * s_n + 1:].view(s_n, nb)
+        self._cu_q, self._ctx_start = on_dev[:s_n + 1], on_dev[s_n + 1:2 * s_n + 1]
+        self._block_tables = on_dev[2 * s_n + 1:].view(s_n, nb)
         if dev.type == "cuda":
             # Positions and slots of the new tokens, made where the tables are. Everything is in
             # place when the constructor returns, on whatever stream it is used then.
-            self.positions, self.slot_mapping, self.last_index = paged_ops.prefill_index(
-                self.cu_q, self.ctx_start, self.block_tables, n_tok, self.max_q_len, cache.block_size)
+            self.positions, self._slot_mapping, self.last_index = paged_ops.prefill_index(
+                self._cu_q, self._ctx_start, self._block_tables, n_tok, self._max_q_len, cache.block_size)
             torch.cuda.current_stream(dev).synchronize()
         else:
             self.positions = torch.from_numpy(np.concatenate(
                 [np.arange(a, a + n, dtype=np.int64) for a, n in zip(self.starts, self.lengths)]))
-            self.slot_mapping = cache.slot_mapping(self.slots, self.starts, self.lengths)
+            self._slot_mapping = cache.slot_mapping(self.slots, self.starts, self.lengths)
             self.last_index = torch.tensor(self.lengths).cumsum(0) - 1
         self._mask_built = False
         self._mask = None
@@ -622,8 +616,8 @@ class PackedPrefillContext:
     def calls(self) -> paged_ops.PrefillStepCalls:
         """The step's layer calls: the shared arguments are checked on the first layer only."""
         if self._calls is None:
-            self._calls = paged_ops.PrefillStepCalls(self.block_tables, self.cu_q, self.ctx_start, self.slot_mapping,
-                                                     self.max_q_len, 1.0 / (self.cache.head_dim ** 0.5))
+            self._calls = paged_ops.PrefillStepCalls(self._block_tables, self._cu_q, self._ctx_start, self._slot_mapping,
+                                                     self._max_q_len, 1.0 / (self.cache.head_dim ** 0.5))
         return self._calls
 
     def attend(self, layer_idx: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:

@@ -11,7 +11,7 @@ from __future__ import annotations
 
 import torch
 import torch.overrides
-from torch.fx._symbolic_trace import is_fx_tracing as _is_fx_tracing
+from torch.fx._symbolic_trace import is_fx_symbolic_tracing
 from torch.utils._device import DeviceContext
 
 from . import _native
@@ -34,7 +34,7 @@ def _observed() -> bool:
     return (torch.compiler.is_compiling()  # first: a compiler that traces this function stops reading here
             or _function_mode() or torch._C._len_torch_dispatch_stack() > 0
             or torch._C._functorch.peek_interpreter_stack() is not None or _FWD_AD._current_level >= 0
-            or torch._C._get_tracing_state() is not None or _is_fx_tracing() or torch.is_autocast_enabled("cuda"))
+            or torch._C._get_tracing_state() is not None or is_fx_symbolic_tracing() or torch.is_autocast_enabled("cuda"))
 
 
 def _open(x: torch.Tensor) -> bool:

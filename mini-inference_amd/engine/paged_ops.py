@@ -579,13 +579,13 @@ def prefill_index(cu_q: torch.Tensor, ctx_start: torch.Tensor, block_tables: tor
     """
     if not cu_q.dtype == ctx_start.dtype == block_tables.dtype == torch.int32:
         raise ValueError("cu_q, ctx_start and block_tables must be int32")
-    if (ctx_start.dim() != 1 or cu_q.shape != (ctx_start.shape[0] + 1,) or block_tables.dim() != 2
-            or block_tables.shape[0] < ctx_start.shape[0] or n_tokens < 0 or max_q_len < 0):
+    s = ctx_start.numel()
+    if (ctx_start.dim() != 1 or cu_q.dim() != 1 or cu_q.numel() != s + 1 or block_tables.dim() != 2
+            or block_tables.size(0) < s or n_tokens < 0 or max_q_len < 0):
         raise ValueError("prefill_index: the step's tensors do not match")
     if not (cu_q.is_contiguous() and ctx_start.is_contiguous()) or block_tables.stride(1) != 1:
         raise ValueError("cu_q, ctx_start and the block_tables rows must be contiguous")
     _require_device(cu_q, ctx_start, block_tables)
-    s = ctx_start.shape[0]
     out = torch.empty(2 * n_tokens + s, dtype=torch.int64, device=cu_q.device)
     positions, slots, last = out[:n_tokens], out[n_tokens:2 * n_tokens], out[2 * n_tokens:]
     if s:
